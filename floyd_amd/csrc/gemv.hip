@@ -259,6 +259,24 @@ int gemv_rows_per_block(const GemvPlan &plan, bool dual) {
 }
 
 bool gemv_mfma(const GemvParams &p, hipStream_t stream, std::string *name = nullptr);  // gemv_mfma.hip
+bool gemv_batch(const GemvParams &p, hipStream_t stream, std::string *name = nullptr);  // gemv_batch.hip
+
+static bool aligned16(const void *ptr) { return ((uintptr_t)ptr & 15u) == 0; }
+
+// Whether the vector kernel takes p's shape and pointers.
+static bool vector_takes(const GemvParams &p) {
+    return row_bytes_of(p.fmt, p.I) % 16 == 0 && (p.fmt != kQ4 || p.I % 2 == 0) &&
+           gemv_lds_bytes_rt(p.fmt, 1, p.I) <= kMaxGemvLds && aligned16(p.w) &&
+           (!p.w2 || aligned16(p.w2)) && aligned16(p.x) && p.x_stride % 4 == 0 &&
+           (!p.norm_w || aligned16(p.norm_w));
+}
+
+// One token row that the matrix-core kernels of gemv_mfma.hip do not take
+// stays on the vector kernel where that can run (q8 2048 x 1408: 3.44 against
+// 3.62 us on the batch kernel; at 2 rows 4.53 against 3.75).
+static bool vector_first(const GemvParams &p, bool vector_ok) {
+    return p.fmt == kF32 || (p.rows == 1 && vector_ok);
+}
 
 // Template name of the kernel gemv() launches for this shape (aligned
 // operands, no pre-split x).
@@ -270,15 +288,15 @@ std::string gemv_kernel_name(int fmt, int O, int I, int rows, bool dual) {
     q.rows = rows;
     q.epilogue = dual ? kEpiSiluDual : q.epilogue;
     std::string mfma;
-    if (gemv_mfma(q, nullptr, &mfma)) return mfma;
+    q.x_stride = I;
+    if (gemv_mfma(q, nullptr, &mfma) || (!vector_first(q, vector_takes(q)) && gemv_batch(q, nullptr, &mfma)))
+        return mfma;
     const GemvPlan pl = plan_gemv(fmt, O, I, rows < kMaxGemvRows ? rows : kMaxGemvRows, dual);
     char buf[96];
     snprintf(buf, sizeof(buf), "mlh::gemv_kernel<0, %d, %d, %d, %d, %d, %d, %d>", fmt, pl.b,
              pl.kt, pl.lpr, pl.r, pl.ks, pl.waves);
     return buf;
 }
-
-static bool aligned16(const void *ptr) { return ((uintptr_t)ptr & 15u) == 0; }
 
 int gemv(const GemvParams &p_in, hipStream_t stream) {
     if (!p_in.w || !p_in.x || !p_in.y || p_in.O <= 0 || p_in.I <= 0 || p_in.rows <= 0)
@@ -297,12 +315,9 @@ int gemv(const GemvParams &p_in, hipStream_t stream) {
     if (gemv_mfma(p_in, stream))
         return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
     if (p_in.router_parts) return kErrArgs;
-    const long row_bytes = row_bytes_of(p_in.fmt, p_in.I);
-    const bool vector_ok =
-        row_bytes % 16 == 0 && (p_in.fmt != kQ4 || p_in.I % 2 == 0) &&
-        gemv_lds_bytes_rt(p_in.fmt, 1, p_in.I) <= kMaxGemvLds && aligned16(p_in.w) &&
-        (!p_in.w2 || aligned16(p_in.w2)) && aligned16(p_in.x) && p_in.x_stride % 4 == 0 &&
-        (!p_in.norm_w || aligned16(p_in.norm_w));
+    const bool vector_ok = vector_takes(p_in);
+    if (!vector_first(p_in, vector_ok) && gemv_batch(p_in, stream))
+        return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
     // token rows beyond 4 run as slices of 4 (register budget) along grid.y
     // of one launch
     bool done = false;

@@ -911,19 +911,25 @@ bool to_host(MoonlightSession *s, void *dst, const void *src, size_t bytes) {
     return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream_of(s)) == hipSuccess;
 }
 
-// Batches of at least this many token rows take the int8-MFMA GEMM (weights
-// read once per 32 or 128 rows) instead of the GEMV (once per 4 rows).  The
-// MoE layer switches at 3 rows: the grouped GEMM streams each active
-// expert once for all its rows in one launch per stage, with the routing in
-// its first launch, while the grouped GEMV runs a routing launch, two stage
-// launches and a combine (measured on MI355X, whole layer: equal at T = 2,
-// 53.5 us; 58 against 74 us at T = 3, 64 against 92 us at T = 4).  The
-// dense projections keep the GEMV up to 16 rows.
+// The MoE layer takes the int8-MFMA GEMM from 3 rows: the grouped GEMM streams
+// each active expert once for all its rows in one launch per stage, with the
+// routing in its first launch, while the grouped GEMV runs a routing launch,
+// two stage launches and a combine (measured on MI355X, whole layer: equal at
+// T = 2, 53.5 us; 58 against 74 us at T = 3, 64 against 92 us at T = 4).
+// The dense projections take it where the batch kernel (gemv_batch.hip, one
+// launch, x split in every workgroup) would need more than kBatchMaxGroups
+// workgroups of 64 weight rows, 16 token rows and 2048 columns: two rounds of
+// the CUs.
 constexpr int kGemmMinRows = 16;
 constexpr int kMoeGemmMinRows = 3;
+constexpr long kBatchMaxGroups = 512;
 
-bool use_gemm(const MoonlightSession *s, int fmt, int rows, int in_w) {
-    return rows >= kGemmMinRows && s->aq && in_w <= s->aq_width && qgemm_shape_ok(fmt, in_w);
+// out_w: weight rows of the launch (a SwiGLU pair: gate and up).
+bool use_gemm(const MoonlightSession *s, int fmt, int rows, int in_w, int out_w) {
+    if (rows < kGemmMinRows || !s->aq || in_w > s->aq_width || !qgemm_shape_ok(fmt, in_w))
+        return false;
+    const long groups = ((long)out_w + 63) / 64 * ((rows + 15) / 16) * ((in_w + 2047) / 2048);
+    return groups > kBatchMaxGroups;
 }
 
 int gemm_rows(MoonlightSession *s, const Matrix &m, const Matrix *up, const float *x, int rows,
@@ -964,7 +970,7 @@ struct RouterFuse {
 int gemv_rows(MoonlightSession *s, const Matrix &m, const float *x, int rows, int in_w,
               int out_w, float *y, const float *norm_w = nullptr, const float *resid = nullptr,
               const RouterFuse *rf = nullptr) {
-    if (!rf && use_gemm(s, m.fmt, rows, in_w))
+    if (!rf && use_gemm(s, m.fmt, rows, in_w, out_w))
         return gemm_rows(s, m, nullptr, x, rows, in_w, out_w, y, norm_w, resid);
     GemvParams p;
     p.fmt = m.fmt;
@@ -993,7 +999,7 @@ int gemv_rows(MoonlightSession *s, const Matrix &m, const float *x, int rows, in
 
 int swiglu_rows(MoonlightSession *s, const Matrix &g, const Matrix &u, const float *x, int rows,
                 int in_w, int width, float *h, const float *norm_w) {
-    if (g.fmt == u.fmt && use_gemm(s, g.fmt, rows, in_w))
+    if (g.fmt == u.fmt && use_gemm(s, g.fmt, rows, in_w, 2 * width))
         return gemm_rows(s, g, &u, x, rows, in_w, width, h, norm_w, nullptr);
     GemvParams p;
     p.fmt = g.fmt;
