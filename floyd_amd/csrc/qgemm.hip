@@ -4,9 +4,9 @@
 // Workgroup: 8 waves in a 4 x 2 arrangement over a 128 (token rows) x 256
 // (weight rows) tile; each wave owns 32 x 128 = 1 x 4 MFMA blocks per limb
 // (three limbs: 192 int32 accumulators, two waves per SIMD).  Pipeline: q8
-// has three LDS stages of 64-wide k slices copied straight into LDS by
-// global_load_lds, two in flight while one is multiplied; q4 has two stages,
-// 64-wide slices unpacked in registers on the way.  One barrier per slice.
+// k slices are 128 wide and copied straight into LDS by buffer loads, one in
+// flight while one is multiplied; q4 slices are 64 wide and unpacked in
+// registers on the way.  One barrier per slice.
 // MFMA operand layout (measured on gfx950): lane l supplies row (l % 32) and
 // the 16-byte k chunk (l / 32) of a 32-wide k step, for A rows and for B
 // columns alike; result register r of lane l is
@@ -284,12 +284,12 @@ __device__ __forceinline__ bool map_tile(const QGemmLaunch &L, GemmTask &tk, int
 // so that the MFMA fragment reads (32 consecutive rows, one chunk) and the
 // tile writes hit distinct banks whether the LDS serves 8 or 16 lanes of a
 // 128-bit access per cycle.
-// Stage width: q8 32-row tiles (weight-stream bound) copy 128-k slices, so a
-// DMA instruction covers 8 rows x 128 contiguous bytes (on MI355X runs of
-// 128 bytes stream ~6 TB/s, runs of 64 bytes ~4.2 TB/s); the 128-row tile
-// (MFMA bound) keeps 64-k slices to fit more stages.
+// q8 slices are 128 k wide, so a DMA instruction covers 8 rows x 128 contiguous
+// bytes (on MI355X runs of 128 bytes stream ~6 TB/s, runs of 64 bytes ~4.2
+// TB/s; the 128-row tile's fill alone took 2300 clocks a 64-k share against
+// 2900).  The 128-row tile's two stages fill the LDS.
 template <int FMT, int BM> struct QgCfg {
-    static constexpr int kRB = (FMT == kQ8 && BM == 32) ? 128 : 64;
+    static constexpr int kRB = FMT == kQ8 ? 128 : 64;
 };
 
 template <int RB>
@@ -315,11 +315,12 @@ template <int FMT, int BM> struct QgShape {
     static constexpr int kWN = kWaves / kWM;       // waves along the weight rows
     static constexpr int kMI = 1;
     static constexpr int kNF = kQgBW / 32 / kWN;   // 32-row weight blocks per wave
-    static constexpr int kStages = FMT == kQ8 ? 3 : 2;
+    static constexpr int kStages = FMT == kQ8 && BM == 32 ? 3 : 2;
     static constexpr int kLdsA = kLimbs * BM * kRB;
     static constexpr int kStage = (kLimbs * BM + kQgBW) * kRB;
-    static constexpr int kLds = kStages * kStage + BM * 8;  // + scales and row map
+    static constexpr int kLds = kStages * kStage;
     static constexpr int kRowBlocks = BM / kRowsDma;
+    static constexpr int kAOffs = kRowBlocks > kWaves ? kRowBlocks / kWaves : 1;  // A row blocks per wave
     static constexpr int kABlocks = kLimbs * kRowBlocks;
     static constexpr int kBBlocks = kQgBW / kRowsDma;
     static constexpr int kBPer = kBBlocks / kWaves;
@@ -328,7 +329,7 @@ template <int FMT, int BM> struct QgShape {
     // register path (q4): 16-byte A chunks and packed B chunks per thread and slice
     static constexpr int kNA = (kLimbs * BM * 4 + kThreads - 1) / kThreads;
     static constexpr int kNB = kQgBW * 2 / kThreads;
-    static_assert(kWaves % kRowBlocks == 0 || kRowBlocks % kWaves == 0, "A row block per wave");
+    static_assert(kWaves % kRowBlocks == 0 || kRowBlocks % kWaves == 0, "A row blocks of a wave");
     static_assert(kBBlocks % kWaves == 0 && (kQgBW * 2) % kThreads == 0, "B split");
 };
 static_assert(QgShape<kQ8, kQgBM>::kLds <= 160 * 1024, "q8 128-row tile exceeds the LDS");
@@ -339,6 +340,41 @@ static_assert(2 * QgShape<kQ4, kQgBMSmall>::kLds <= 160 * 1024, "two q4 32-row t
 // 3:0 and 15:14, expcnt 6:4 and lgkmcnt 11:8 left at their no-wait maxima).
 template <int N> __device__ __forceinline__ void wait_vmcnt() {
     __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+
+// Buffer of `bytes` from base: loads at offsets of that and more read zero,
+// stores there are dropped.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *base, long bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0,
+                                             bytes < 0xFFFFFFFFL ? (unsigned)bytes : 0xFFFFFFFFu, 0x00027000);
+}
+// 16 bytes per lane from voffset + soffset to consecutive LDS bytes.
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t buf, unsigned voffset, int soffset,
+                                      __attribute__((address_space(3))) int8_t *dst) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, dst, 16, voffset, soffset, 0, 0);
+}
+__device__ __forceinline__ float buffer_load_f32(__amdgpu_buffer_rsrc_t buf, unsigned voffset) {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(buf, voffset, 0, 0));
+}
+__device__ __forceinline__ void buffer_store_f32(__amdgpu_buffer_rsrc_t buf, float v, unsigned voffset) {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), buf, voffset, 0, 0);
+}
+
+// silu(g) * u = g u / (1 + e^-g) in a third of the instructions of expf and an
+// IEEE division, to the same error (1.5 ulp): e^-g = 2^t with the rounding of
+// t = -g log2(e) carried into the result, the quotient by a reciprocal and one
+// remainder step.  g is held at -87 and above (silu there is under 2e-36), so
+// that e^-g and its reciprocal stay in fp32's normal range; NaN stays NaN.
+__device__ __forceinline__ float silu_times(float g, float u) {
+    constexpr float kLog2e = 1.44269504f, kLog2eRest = 1.92596299e-8f, kLn2 = 0.693147181f;
+    g = __builtin_elementwise_maximum(g, -87.0f);
+    const float t = -g * kLog2e;
+    const float rest = fmaf(-g, kLog2eRest, fmaf(-g, kLog2e, -t));
+    const float p = __builtin_amdgcn_exp2f(t);
+    const float d = 1.0f + fmaf(p, rest * kLn2, p);
+    const float r = __builtin_amdgcn_rcpf(d), n = g * u;
+    const float q = n * r;
+    return fmaf(fmaf(-d, q, n), r, q);
 }
 
 // Workgroup over a BM x 256 tile (QgShape).  The 32-row tile serves
@@ -356,8 +392,7 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
     constexpr int kLdsA = Sh::kLdsA;
     constexpr int kMI = Sh::kMI, kNF = Sh::kNF;
     constexpr bool kDma = FMT == kQ8;
-    float *lds_scale = reinterpret_cast<float *>(qg_lds + kStages * kStage);
-    int *lds_arow = reinterpret_cast<int *>(qg_lds + kStages * kStage + BM * 4);
+    float *lds_scale = reinterpret_cast<float *>(qg_lds);  // after the products
     GemmTask tk;
     int m0, n0;
     if (!map_tile<DUAL, BM>(L, tk, m0, n0)) return;
@@ -379,18 +414,11 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
     const bool live =
         Sh::kWM == 1 || __builtin_amdgcn_readfirstlane(m0 + wm * (Sh::kMI * 32)) < tk.rows;
 
-    if (tid < BM) {
-        const int m = m0 + tid;
-        int arow = -1;
-        float sc = 0.0f;
-        if (m < tk.rows) {
-            arow = tk.a_rows ? tk.a_rows[m] : m;
-            sc = tk.a_scale[arow];
-        }
-        lds_arow[tid] = arow;
-        lds_scale[tid] = sc;
-    }
-    __syncthreads();
+    // activation row of tile row r (past the task's end: row m0)
+    auto arow_of = [&](int r) {
+        const int m = m0 + r < tk.rows ? m0 + r : m0;
+        return tk.a_rows ? tk.a_rows[m] : m;
+    };
 
     // ---- per-thread global sources (fixed over k).  Rows past the task's end
     // read row m0 (A) or weight row 0 (B): their outputs are never stored.
@@ -425,8 +453,7 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
         return a_base + limb * a_plane;
     };
     auto a_row_src = [&](int limb, int r) -> const int8_t * {
-        const int arow = lds_arow[r] >= 0 ? lds_arow[r] : lds_arow[0];
-        return limb_base(limb) + (long)arow * tk.a_stride;
+        return limb_base(limb) + (long)arow_of(r) * tk.a_stride;
     };
 
     // DMA path (q8), blocks of R = 1024 / kRB rows = 1 KB: A block b holds
@@ -438,8 +465,12 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
     // share a lane's A rows.
     constexpr int kCh = kRB / 16;
     const int lr = lane / kCh, lc = lane % kCh;
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     auto swz = [](int r) { return kRB == 64 ? (((r >> 1) ^ (r >> 3)) & 3) : ((r ^ (r >> 3)) & 7); };
-    unsigned a_off = 0u;  // byte offset of this lane's A row
+    // byte offsets of this lane's A rows; past the task's end outside the
+    // buffer (read as zeros)
+    constexpr long kABytes = 0xF0000000L;
+    unsigned a_off[Sh::kAOffs];
     // register path (q4, 64-byte rows): kNA A chunks and kNB packed B chunks
     constexpr int kNA = Sh::kNA, kNB = Sh::kNB;
     const int8_t *a_src[kNA];
@@ -448,9 +479,11 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
     int b_dst[kNB];
     u32x4 ra[kNA], rb[kNB];
     if constexpr (kDma) {
-        const int r = (wave % Sh::kRowBlocks) * Sh::kRowsDma + lr;
-        const int arow = lds_arow[r] >= 0 ? lds_arow[r] : lds_arow[0];
-        a_off = (unsigned)(arow * tk.a_stride);
+#pragma unroll
+        for (int h = 0; h < Sh::kAOffs; ++h) {
+            const int r = ((wave + Sh::kWaves * h) % Sh::kRowBlocks) * Sh::kRowsDma + lr;
+            a_off[h] = m0 + r < tk.rows ? (unsigned)(arow_of(r) * tk.a_stride) : (unsigned)kABytes;
+        }
     } else {
 #pragma unroll
         for (int q = 0; q < kNA; ++q) {
@@ -468,38 +501,36 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
         }
     }
 
-    // one k slice of 64 into LDS stage buf (kDmaMin or kDmaMax DMA
-    // instructions per wave)
+    // one k slice into LDS stage buf (kDmaMin or kDmaMax DMA instructions per
+    // wave).  Buffer loads: with a flat LDS DMA in flight the compiler makes
+    // every wait for an LDS read a wait for all of them.  Weight rows past
+    // the task's last are out of the buffer's range and arrive as zeros.
     auto issue_dma = [&](int k0, int buf) {
         __attribute__((address_space(3))) int8_t *stage =
             (__attribute__((address_space(3))) int8_t *)(qg_lds + buf * kStage);
         constexpr int kRowBlocks = Sh::kRowBlocks;
 #pragma unroll
         for (int h = 0; h < Sh::kAMax; ++h) {
-            const int b = wave + Sh::kWaves * h;  // A block
+            const int b = wave_u + Sh::kWaves * h;  // A block
             if (h >= Sh::kAMin && b >= Sh::kABlocks) break;  // wave-uniform
             const int limb = b / kRowBlocks, rb = b % kRowBlocks;
-            const int r = rb * Sh::kRowsDma + lr;  // A row of this lane
-            const int ca = lc ^ swz(r);
-            // uniform base + 32-bit lane offset: one VGPR per address
-            const unsigned aoff = a_off + (unsigned)(k0 + ca * 16);
-            __builtin_amdgcn_global_load_lds(
-                (const __attribute__((address_space(1))) void *)(limb_base(limb) + aoff),
-                stage + b * 1024, 16, 0, 0);
+            const int chunk = lc ^ swz(rb * Sh::kRowsDma + lr);
+            // a reduction that ends inside the slice: zeros past it
+            const bool past = k0 + kRB > tk.k && k0 + chunk * 16 >= tk.k;
+            dma16(buffer_of(limb_base(limb), kABytes),
+                  past ? (unsigned)kABytes : a_off[h % Sh::kAOffs] + (unsigned)(chunk * 16), k0,
+                  stage + b * 1024);
         }
 #pragma unroll
         for (int q = 0; q < Sh::kBPer; ++q) {
-            const int bb = wave + Sh::kWaves * q;
+            const int bb = wave_u + Sh::kWaves * q;
             const int j = bb * Sh::kRowsDma + lr;  // B row of this lane
             bool up;
-            const int out = b_out(j, up);
-            const uint8_t *bbase = up ? w_up : w_gate;
-            const int cb = lc ^ swz(j);
-            const unsigned boff =
-                (unsigned)((out < tk.n_out ? out : 0) * w_row_bytes) + (unsigned)(k0 + cb * 16);
-            __builtin_amdgcn_global_load_lds(
-                (const __attribute__((address_space(1))) void *)(bbase + boff),
-                stage + kLdsA + bb * 1024, 16, 0, 0);
+            (void)b_out(bb * Sh::kRowsDma, up);  // a block's rows are of one matrix
+            bool u;
+            dma16(buffer_of(up ? w_up : w_gate, tk.n_out * w_row_bytes),
+                  (unsigned)(b_out(j, u) * w_row_bytes) + (unsigned)((lc ^ swz(j)) * 16), k0,
+                  stage + kLdsA + bb * 1024);
         }
     };
     auto fetch = [&](int k0) {
@@ -575,34 +606,94 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
                             fa[s2][a][i], fb[s2][f], acc[a][i][f], 0, 0, 0);
     };
 
+    // LDS byte of this lane's first A / B fragment.  Steps and blocks differ
+    // from it by an xor of bits 5 and 6 (lds_off: 16-byte chunk 2 st + half,
+    // swizzled by the row; 32 rows on flips the swizzle's top bit) and by
+    // constants, computed where used: kept over the loop they would spill
+    const int a_frag = lds_off<kRB>(wm * (kMI * 32) + frow, half);
+    const int b_frag = kLdsA + lds_off<kRB>(wn * (kNF * 32) + frow, half);
     if constexpr (kDma) {
-        // kStages stages: slices ks + 1 .. ks + kStages - 1 stream into LDS
-        // while slice ks is multiplied.  A wave's DMA completes in order, its
-        // kDmaMax or kDmaMin instructions per slice, so slice ks has landed
-        // when at most that many for the later slice in flight remain; the
-        // barrier after the wait makes every wave's part visible and frees
-        // the stage of slice ks - 1 for slice ks + kStages - 1.
-        static_assert(kStages == 3, "waits below assume one later slice in flight");
-        const bool more = Sh::kDmaMax == Sh::kDmaMin ||
-                          __builtin_amdgcn_readfirstlane(wave) + Sh::kWaves * Sh::kAMin <
-                              Sh::kABlocks;
-        const int nk = tk.k / kRB;  // k % kRB == 0 (qgemm_shape_ok, and the tile pickers for kRB = 128)
-        for (int st = 0; st < kStages - 1 && st < nk; ++st) issue_dma(st * kRB, st);
-        for (int ks = 0; ks < nk; ++ks) {
-            if (ks + 1 < nk) {
+        // Slices ks + 1 .. ks + kStages - 1 stream into LDS while slice ks is
+        // multiplied.  A wave's DMA completes in order, its kDmaMax or
+        // kDmaMin instructions per slice, so a slice has landed when at most
+        // that many for each later slice in flight remain; the barrier after
+        // the wait makes every wave's part visible and frees the stage of the
+        // slice before it.  (A bare barrier: __syncthreads() would also wait
+        // for the loads of the fence it implies.)
+        static_assert(kStages == 2 || kStages == 3, "waits below");
+        const bool more = Sh::kDmaMax == Sh::kDmaMin || wave_u + Sh::kWaves * Sh::kAMin < Sh::kABlocks;
+        const int nk = (tk.k + kRB - 1) / kRB;
+        // slice ks has landed for every wave, and the stage of slice ks - 1 is
+        // free: it takes slice ks + kStages - 1
+        auto next_slice = [&](int ks) {
+            if (kStages == 3 && ks + 1 < nk) {
                 if (more) wait_vmcnt<Sh::kDmaMax>();
                 else wait_vmcnt<Sh::kDmaMin>();
             } else {
                 wait_vmcnt<0>();
             }
-            // a bare barrier: __syncthreads() would also wait for the stores
-            // and loads of the fence it implies
             __builtin_amdgcn_s_barrier();
             if (ks + kStages - 1 < nk) issue_dma((ks + kStages - 1) * kRB, (ks + kStages - 1) % kStages);
-            if (live) {
+        };
+        // Fragments are read ahead of their products, the weights by two
+        // blocks and the activations by a step.  The sched_barriers keep the
+        // order: left to itself the compiler reads a block, waits for it and
+        // multiplies it, because the accumulators leave it few registers.
+        // (Reading ahead across slices too, the barrier two blocks before a
+        // slice's end: the T = 2048 q8 MoE layer 568 against 557 us.)  T = 2048 q8 MoE gate / up
+        // 350 -> 282 us with 128-wide slices, buffer DMA and this order.
+        constexpr int kSteps = kRB / 32, kBlocks = kSteps * kNF;
+        static_assert(kBlocks % 4 == 0 && kSteps % 2 == 0, "register rings");
+        i32x4 fa[2][kLimbs], fb[4];
+        auto read_a = [&](int base, int st, int a) {
+            fa[st & 1][a] = *reinterpret_cast<const i32x4 *>(qg_lds + ((base + a_frag) ^ (st % kSteps << 5)) +
+                                                             a * (BM * kRB));
+        };
+        auto read_b = [&](int base, int i) {
+            const int st = i / kNF, f = i % kNF;
+            fb[i % 4] = *reinterpret_cast<const i32x4 *>(
+                qg_lds + ((base + b_frag) ^ ((st << 5) ^ ((f & 1) << 6))) + f * 32 * kRB);
+        };
+        for (int st = 0; st < kStages - 1 && st < nk; ++st) issue_dma(st * kRB, st);
+        next_slice(0);
+        if (live) {
+            int base = 0;
 #pragma unroll
-                for (int kp = 0; kp < kRB / 32; kp += 2) compute_pair(ks % kStages, kp);
+            for (int a = 0; a < kLimbs; ++a) read_a(0, 0, a);
+            read_b(0, 0);
+            read_b(0, 1);
+            for (int ks = 0; ks < nk; ++ks) {
+                asm("" : "+s"(base));  // (see a_frag)
+                const int next = (ks + 1) % kStages * kStage;
+                if (ks) {
+                    next_slice(ks);
+#pragma unroll
+                    for (int a = 0; a < kLimbs; ++a) read_a(base, 0, a);
+                    read_b(base, 0);
+                    read_b(base, 1);
+                }
+#pragma unroll
+                for (int i = 0; i < kBlocks; ++i) {
+                    const int st = i / kNF, f = i % kNF;
+                    if (i + 2 < kBlocks) {
+                        read_b(base, i + 2);
+                    }
+                    if (st + 1 < kSteps) {
+                        constexpr int per = (kLimbs + kNF - 1) / kNF;
+#pragma unroll
+                        for (int a = f * per; a < (f + 1) * per && a < kLimbs; ++a) read_a(base, st + 1, a);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int a = 0; a < kLimbs; ++a)
+                        acc[a][0][f] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[st & 1][a], fb[i % 4],
+                                                                             acc[a][0][f], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                base = next;
             }
+        } else {
+            for (int ks = 1; ks < nk; ++ks) next_slice(ks);
         }
     } else {
         // two buffers: slice ks + 2 is in registers while slice ks is multiplied
@@ -621,83 +712,64 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
         }
     }
 
-    // ---- epilogue.  Every global input of the epilogue (weight scales,
-    // residual rows) is loaded before the first store: the stores may alias
-    // them as far as the compiler knows, so a load after a store would wait
-    // for it.
+    // ---- epilogue, without a branch: stores and residual loads go through
+    // buffers of the tile's own rows, so rows past the task's end are out of
+    // range (dropped, read as zero), as are the columns past n_out, whose
+    // offset is set there.  Weight scales and residual rows are loaded before
+    // the stores they precede: a wait for a load after a store waits for both.
     constexpr int kF = DUAL ? kNF / 2 : kNF;
+    constexpr unsigned kOutside = 0x7FFFFFFFu;
+    const int rows_here = min(tk.rows - m0, BM);
     float sw[kF], su[kF];
-    int ncol[kF];
+    unsigned ycol[kF], rcol[kF];
+    const auto s_buf = buffer_of(tk.s, (long)tk.n_out * 4);
+    const auto s2_buf = buffer_of(DUAL ? tk.s2 : tk.s, (long)tk.n_out * 4);
+    const auto y_buf = buffer_of(tk.y + (long)m0 * tk.y_stride, (long)rows_here * tk.y_stride * 4);
+    const int lane_row = wm * (kMI * 32) + half * 4;  // + 8 (r / 4) + r % 4: row of result register r
 #pragma unroll
     for (int f = 0; f < kF; ++f) {
-        ncol[f] = n0 + wn * kF * 32 + f * 32 + frow;
-        const bool ok = ncol[f] < tk.n_out;
-        sw[f] = ok ? load_global_f32(tk.s + ncol[f]) : 0.0f;
-        su[f] = (DUAL && ok) ? load_global_f32(tk.s2 + ncol[f]) : 0.0f;
+        const int n = n0 + wn * kF * 32 + f * 32 + frow;
+        sw[f] = buffer_load_f32(s_buf, n * 4);
+        su[f] = DUAL ? buffer_load_f32(s2_buf, n * 4) : 0.0f;
+        ycol[f] = n < tk.n_out ? (unsigned)(lane_row * tk.y_stride + n) * 4 : kOutside;
+        rcol[f] = n < tk.n_out ? (unsigned)(lane_row * tk.resid_stride + n) * 4 : kOutside;
     }
-    // row scales of the result rows this lane holds
-    float sxr[kMI][16];
-#pragma unroll
-    for (int i = 0; i < kMI; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-            sxr[i][r] = lds_scale[wm * (kMI * 32) + i * 32 + (r >> 2) * 8 + half * 4 + (r & 3)];
-    // complete the scale loads now: stores share the vector-memory counter,
-    // so a wait placed after the first store would also wait for the stores
-    __builtin_amdgcn_s_waitcnt(0);
+    // every wave has read its last fragments: the LDS takes the row scales
+    __syncthreads();
+    if (tid < BM) lds_scale[tid] = tid < rows_here ? tk.a_scale[arow_of(tid)] : 0.0f;
+    __syncthreads();
     // 65536 hi + 256 mid + lo of one result register (the int32 sums are exact)
-    auto limb_sum = [&](int i, int f, int r) -> float {
-        return (float)acc[0][i][f][r] * 65536.0f +
-               ((float)acc[1][i][f][r] * 256.0f + (float)acc[2][i][f][r]);
+    auto limb_sum = [&](int f, int r) -> float {
+        return fmaf((float)acc[0][0][f][r], 65536.0f,
+                    fmaf((float)acc[1][0][f][r], 256.0f, (float)acc[2][0][f][r]));
     };
-    // the residual and plain paths are separate instantiations, so the plain
-    // path carries no wait for residual loads (which would drain the stores)
     auto epilogue = [&](auto with_resid) {
         constexpr bool kResid = decltype(with_resid)::value;
+        const auto r_buf = buffer_of(kResid ? tk.resid + (long)m0 * tk.resid_stride : tk.y,
+                                     (long)rows_here * tk.resid_stride * 4);
 #pragma unroll
-        for (int i = 0; i < kMI; ++i) {
+        for (int rg = 0; rg < 4; ++rg) {
+            const f32x4 sx = *reinterpret_cast<const f32x4 *>(lds_scale + lane_row + 8 * rg);
+            float res[4][kF];
+            if (kResid) {
 #pragma unroll
-            for (int rg = 0; rg < 16; rg += 4) {
-                // residual inputs of 4 result registers, loaded before their stores
-                float res[4][kF];
-                if (kResid) {
+                for (int q = 0; q < 4; ++q)
 #pragma unroll
-                    for (int r = rg; r < rg + 4; ++r) {
-                        const int m = m0 + wm * (kMI * 32) + i * 32 + (r >> 2) * 8 + half * 4 + (r & 3);
+                    for (int f = 0; f < kF; ++f)
+                        res[q][f] = buffer_load_f32(
+                            r_buf, rcol[f] + (unsigned)((8 * rg + q) * tk.resid_stride * 4));
+            }
 #pragma unroll
-                        for (int f = 0; f < kF; ++f)
-                            res[r - rg][f] = (m < tk.rows && ncol[f] < tk.n_out)
-                                                 ? load_global_f32(tk.resid +
-                                                                   (long)m * tk.resid_stride +
-                                                                   ncol[f])
-                                                 : 0.0f;
-                    }
-                }
+            for (int q = 0; q < 4; ++q) {
+                const int r = 4 * rg + q;
+                const float s = q == 0 ? sx.x : q == 1 ? sx.y : q == 2 ? sx.z : sx.w;
+                const unsigned row = (unsigned)((8 * rg + q) * tk.y_stride * 4);
 #pragma unroll
-                for (int r = rg; r < rg + 4; ++r) {
-                    const int m = m0 + wm * (kMI * 32) + i * 32 + (r >> 2) * 8 + half * 4 + (r & 3);
-                    if (m >= tk.rows) continue;
-                    const float sx = sxr[i][r];
-                    float *yrow = tk.y + (long)m * tk.y_stride;
-                    if (DUAL) {
-#pragma unroll
-                        for (int f = 0; f < kF; ++f) {
-                            if (ncol[f] < tk.n_out) {
-                                const float g = limb_sum(i, f, r) * sx * sw[f];
-                                const float u = limb_sum(i, f + kF, r) * sx * su[f];
-                                store_global(yrow + ncol[f], silu(g) * u);
-                            }
-                        }
-                    } else {
-#pragma unroll
-                        for (int f = 0; f < kF; ++f) {
-                            if (ncol[f] < tk.n_out) {
-                                float v = limb_sum(i, f, r) * sx * sw[f];
-                                if (kResid) v = res[r - rg][f] + v;
-                                store_global(yrow + ncol[f], v);
-                            }
-                        }
-                    }
+                for (int f = 0; f < kF; ++f) {
+                    float v = limb_sum(f, r) * s * sw[f];
+                    if (DUAL) v = silu_times(v, limb_sum(f + kF, r) * s * su[f]);
+                    if (kResid) v = res[q][f] + v;
+                    buffer_store_f32(y_buf, v, ycol[f] + row);
                 }
             }
         }
@@ -987,28 +1059,25 @@ static int tile_bm(int kind) {
 }
 
 // Tile choices, measured on MI355X.  A batch of at most 16 token rows streams
-// the weights (every task fits one row tile); the streaming tile and the q8
-// 32-row tile copy 128 k per step, so they need reductions that are whole
-// multiples of 128 (`k128`; otherwise the 128-row tile runs).
+// the weights (every task fits one row tile); the streaming tile needs
+// reductions that are whole multiples of 128 (`k128`).
 // MoE layer: 16-row streaming tile up to 16 rows (T = 8: 99 against 108 us
 // on the 32-row LDS tile), the 32-row LDS tile up to 80 rows per expert on
 // average (T = 64: 170 against 180 us streaming), 128 rows above.  Dense
 // projections: the 32-row tile up to 64 rows.
-static int moe_tile(int fmt, int rows, double rows_per_expert, bool k128) {
+static int moe_tile(int rows, double rows_per_expert, bool k128) {
     if (k128 && rows <= 16) return kTileStream16;
-    const bool small_ok = fmt == kQ4 || k128;  // the q8 32-row tile steps 128 k
-    return small_ok && rows_per_expert <= 80.0 ? kTileLds32 : kTileLds128;
+    return rows_per_expert <= 80.0 ? kTileLds32 : kTileLds128;
 }
 // Dense projections whose 128-row tiles would cover at most half the CUs
 // (o_proj and the dense down projection at 2048 rows: 128 tiles) take the
 // 32-row tile too: 52.8 against 58.4 us for o_proj at 2048 rows; at 240
 // tiles (`[q; kv_a]`) the 32-row tile measured 75.1 against 51.1 us.
-static int dense_tile(int fmt, int rows, bool k128, int n_out, bool dual) {
+static int dense_tile(int rows, bool k128, int n_out, bool dual) {
     if (k128 && rows <= 16) return kTileStream16;
-    const bool small_ok = fmt == kQ4 || k128;
     const int outw = dual ? kQgBW / 2 : kQgBW;
     const long t128 = (long)((rows + kQgBM - 1) / kQgBM) * ((n_out + outw - 1) / outw);
-    return small_ok && (rows <= 2 * kQgBMSmall || t128 <= 128) ? kTileLds32 : kTileLds128;
+    return rows <= 2 * kQgBMSmall || t128 <= 128 ? kTileLds32 : kTileLds128;
 }
 
 static int launch_qgemm_fmt(int fmt, bool dual, int kind, const QGemmLaunch &L, int tiles_bound,
@@ -1038,7 +1107,7 @@ int qgemm_single(int fmt, bool dual, const GemmTask &task, hipStream_t stream) {
         return kErrArgs;
     QGemmLaunch L;
     L.single = task;
-    const int kind = dense_tile(fmt, task.rows, task.k % 128 == 0, task.n_out, dual);
+    const int kind = dense_tile(task.rows, task.k % 128 == 0, task.n_out, dual);
     return launch_qgemm_fmt(fmt, dual, kind, L,
                             host_tiles(dual, task.rows, task.n_out, tile_bm(kind)), stream);
 }
@@ -1235,8 +1304,7 @@ int moe_gemm(const MoeGemmParams &p, hipStream_t stream) {
     // one tile kind for the whole layer, from the average rows per expert
     const bool k128 = p.hidden % 128 == 0 && p.inter % 128 == 0 &&
                       (!p.has_shared || p.shared_width % 128 == 0);
-    const bool any_q8 = p.expert_fmt == kQ8 || (p.has_shared && p.shared_fmt == kQ8);
-    const int kind = moe_tile(any_q8 ? kQ8 : kQ4, p.rows, (double)entries / p.experts, k128);
+    const int kind = moe_tile(p.rows, (double)entries / p.experts, k128);
     const int bm = tile_bm(kind);
     MoeScheduleParams sp;
     sp.p = p;
