@@ -31,19 +31,39 @@ constexpr int kQgBK = 64;   // k per pipeline stage
 constexpr int kQgGroup = 4; // row tiles per locality group
 constexpr int kQgMaxTasks = 272;
 
+// Quantised activations lie in blocks of 8 rows x 128 columns: the three limbs'
+// (hi, mid, lo) 8 x 128 bytes one after the other, a row block's column blocks
+// one after the other.  A tile's copy of 8 rows of a limb is then 1 KB in one
+// piece where its rows follow each other (a probe of the tile's fill alone:
+// 1780 clocks a 64-k share from such pieces, 2300 from 128-byte runs of limb
+// planes, 2900 from 64-byte runs).
+constexpr int kLimbBlock = 3 * 8 * 128;
+__host__ __device__ inline long limb_row_block(int width) {  // bytes per 8 rows
+    return (long)((width + 127) / 128) * kLimbBlock;
+}
+__host__ __device__ inline long limb_bytes(long rows, int width) {
+    return (rows + 7) / 8 * limb_row_block(width);
+}
+// Byte of limb 0 at (row, col); limb l is 1024 l further.
+__host__ __device__ inline long limb_at(long row, int col, int width) {
+    return (row >> 3) * limb_row_block(width) + (col >> 7) * kLimbBlock + (row & 7) * 128 + (col & 127);
+}
+
 // One independent product: rows x n_out outputs, reduction length k.
 struct GemmTask {
     const uint8_t *w = nullptr, *w2 = nullptr;  // [n_out][k] packed (w2: up rows, SwiGLU)
     const float *s = nullptr, *s2 = nullptr;    // per weight row scales
     int rows = 0, n_out = 0, k = 0;
     int w_ld = 0;  // weight row length in elements (0: k); a k slice of longer rows
-    // quantised activations: limb l (0 hi, 1 mid, 2 lo) of row r at
-    // a + l * a_plane + r * a_stride
+    // quantised activations (limb blocks), from their first column on (a
+    // multiple of 128); a_width: columns of a whole row
     const int8_t *a = nullptr;
-    long a_plane = 0;
+    int a_width = 0;
     const float *a_scale = nullptr;
-    long a_stride = 0;
-    const int *a_rows = nullptr;  // optional: activation row of token row m
+    // activation row of token row m (of a and a_scale): a_rows[m] if set, else
+    // a_row0 + m
+    const int *a_rows = nullptr;
+    int a_row0 = 0;
     float *y = nullptr;           // output row m at y + m * y_stride
     long y_stride = 0;
     const float *resid = nullptr;  // optional residual (y = resid + product)
@@ -61,10 +81,9 @@ struct QGemmLaunch {
 
 // Per-row activation quantisation (optionally RMSNorm'ed first,
 // moonlight_kernels.metal:23-41): rows of `x` (stride x_stride floats) ->
-// limbs hi, mid, lo at q, q + plane, q + 2 plane (row stride `width` bytes)
-// and scales.
+// limb blocks at q (limb_bytes(rows, width)) and scales.
 int quantize_activations(const float *x, long x_stride, int rows, int width, const float *norm_w,
-                         float eps, int8_t *q, long plane, float *scale, hipStream_t stream);
+                         float eps, int8_t *q, float *scale, hipStream_t stream);
 
 // One dense task, e.g. a prefill projection.  Epilogue: plain or residual
 // (task.resid) or SwiGLU pair (dual, task.w2 = up).
@@ -88,16 +107,12 @@ struct MoeGemmParams {
     const float *x = nullptr;  // residual stream [rows, hidden]
     const float *norm_w = nullptr;
     float eps = 1e-5f;
-    // scratch
-    // three limb planes each (limb l at base + l * plane)
-    int8_t *xq = nullptr;  // [3][rows, hidden]
-    long xq_plane = 0;
+    // scratch: limb blocks and scales
+    int8_t *xq = nullptr;       // [rows, hidden]
     float *xq_scale = nullptr;  // [rows]
-    int8_t *hq = nullptr;  // [3][rows*top_k, inter]
-    long hq_plane = 0;
+    int8_t *hq = nullptr;       // [rows*top_k, inter]
     float *hq_scale = nullptr;  // [rows*top_k]
-    int8_t *sq = nullptr;  // [3][rows, shared_width]
-    long sq_plane = 0;
+    int8_t *sq = nullptr;       // [rows, shared_width]
     float *sq_scale = nullptr;  // [rows]
     GemmTask *tasks = nullptr;                   // [2][kQgMaxTasks]
     int *tile_start = nullptr;                   // [2][kQgMaxTasks + 1]
@@ -107,9 +122,14 @@ struct MoeGemmParams {
     float *shared_hidden = nullptr;  // [rows, shared_width]
     float *shared_out = nullptr;     // [rows, hidden]
     // optional [rows, hidden]: the shared down projection runs as two k
-    // halves (shared_out + shared_out2) when its width is twice inter
+    // halves (shared_out + shared_out2) where moe_shared_splits
     float *shared_out2 = nullptr;
 };
+// Whether the shared down projection can run as two k halves of `inter`
+// columns (each a whole number of limb blocks).
+__host__ __device__ inline bool moe_shared_splits(int inter, int shared_width) {
+    return shared_width == 2 * inter && inter % 128 == 0;
+}
 int moe_gemm(const MoeGemmParams &p, hipStream_t stream);
 
 // Shapes the MFMA path takes (k a multiple of kQgBK, 16-byte aligned rows).

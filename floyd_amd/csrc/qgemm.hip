@@ -3,10 +3,17 @@
 //
 // Workgroup: 8 waves in a 4 x 2 arrangement over a 128 (token rows) x 256
 // (weight rows) tile; each wave owns 32 x 128 = 1 x 4 MFMA blocks per limb
-// (three limbs: 192 int32 accumulators, two waves per SIMD).  Pipeline: q8
-// k slices are 128 wide and copied straight into LDS by buffer loads, one in
-// flight while one is multiplied; q4 slices are 64 wide and unpacked in
-// registers on the way.  One barrier per slice.
+// (three limbs: 192 int32 accumulators, two waves per SIMD).  Pipeline: k
+// slices are 128 wide and copied as stored straight into LDS by buffer loads,
+// one in flight while one is multiplied (q4 weights are unpacked as they are
+// read); one barrier per slice.
+//
+// Bound: the copies (the layer without products 457 us, without copies 474, at
+// 583 in all for q8 at T = 2048) and the card's power limit (the same launches
+// on zero activations: 495 us).  Whole MoE layer on MI355X, T = 2048: q8 653 ->
+// 556 us, q4 618 -> 543; T = 600: q8 323 -> 296, q4 278 -> 225; T = 64: q8 158
+// -> 154, q4 136 -> 121 (64-wide q8 slices by flat LDS DMA, q4 slices unpacked
+// through registers, limb planes and a read-wait-multiply order before).
 // MFMA operand layout (measured on gfx950): lane l supplies row (l % 32) and
 // the 16-byte k chunk (l / 32) of a 32-wide k step, for A rows and for B
 // columns alike; result register r of lane l is
@@ -20,6 +27,7 @@ namespace mlh {
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kLimbs = 3;
 constexpr float kQuantMax = 4194304.0f;  // 2^22: |65536 * hi + 256 * mid + lo| bound
@@ -54,8 +62,7 @@ __device__ __forceinline__ unsigned pack_bytes(int a, int b, int c, int d) {
 constexpr int kQuantRegChunks = 16;
 
 // One set of rows to quantise: x (row stride x_stride, optionally
-// RMSNorm'ed with norm_w) -> limbs hi, mid, lo at q, q + plane, q + 2 plane
-// (row stride width) and scales.
+// RMSNorm'ed with norm_w) -> limb blocks at q and scales.
 struct QuantSeg {
     const float *x = nullptr;
     long x_stride = 0;
@@ -63,7 +70,6 @@ struct QuantSeg {
     const float *norm_w = nullptr;
     float eps = 0.0f;
     int8_t *q = nullptr;
-    long plane = 0;
     float *scale = nullptr;
 };
 
@@ -73,7 +79,6 @@ __device__ __forceinline__ void quantize_row(const QuantSeg &s, int row) {
     const float *x = s.x, *norm_w = s.norm_w;
     const int width = s.width;
     const float eps = s.eps;
-    int8_t *hi = s.q, *mid = s.q + s.plane, *lo = s.q + 2 * s.plane;
     float *scale = s.scale;
     const int lane = threadIdx.x & (kWave - 1);
     const float *xr = x + (long)row * s.x_stride;
@@ -122,9 +127,7 @@ __device__ __forceinline__ void quantize_row(const QuantSeg &s, int row) {
     amax = dpp_wave_max(amax);
     const float inv = amax > 0.0f ? kQuantMax / amax : 0.0f;
     if (lane == 0) scale[row] = amax / kQuantMax;
-    int8_t *hr = hi + (long)row * width;
-    int8_t *mr = mid + (long)row * width;
-    int8_t *lr = lo + (long)row * width;
+    int8_t *qr = s.q + limb_at(row, 0, width);
     for (int c = 0; c < nc; ++c) {
         const int i = (c * kWave + lane) * 4;
         if (i >= width) continue;
@@ -134,9 +137,10 @@ __device__ __forceinline__ void quantize_row(const QuantSeg &s, int row) {
         quant_limbs(t.y, inv, h1, m1, l1);
         quant_limbs(t.z, inv, h2, m2, l2);
         quant_limbs(t.w, inv, h3, m3, l3);
-        *reinterpret_cast<unsigned *>(hr + i) = pack_bytes(h0, h1, h2, h3);
-        *reinterpret_cast<unsigned *>(mr + i) = pack_bytes(m0, m1, m2, m3);
-        *reinterpret_cast<unsigned *>(lr + i) = pack_bytes(l0, l1, l2, l3);
+        int8_t *at = qr + (i >> 7) * kLimbBlock + (i & 127);
+        *reinterpret_cast<unsigned *>(at) = pack_bytes(h0, h1, h2, h3);
+        *reinterpret_cast<unsigned *>(at + 1024) = pack_bytes(m0, m1, m2, m3);
+        *reinterpret_cast<unsigned *>(at + 2048) = pack_bytes(l0, l1, l2, l3);
     }
 }
 
@@ -152,8 +156,7 @@ __global__ __launch_bounds__(256) void quantize_act_kernel(QuantSeg a, QuantSeg 
 }
 
 static bool quant_seg_ok(const QuantSeg &s) {
-    return s.rows == 0 || (s.x && s.q && s.plane >= (long)s.rows * s.width && s.scale &&
-                           s.rows > 0 && s.width > 0 &&
+    return s.rows == 0 || (s.x && s.q && s.scale && s.rows > 0 && s.width > 0 &&
                            s.width % 4 == 0 && s.x_stride % 4 == 0);
 }
 
@@ -172,7 +175,7 @@ static int quantize_segments(const QuantSeg &a, const QuantSeg &b, hipStream_t s
 }
 
 int quantize_activations(const float *x, long x_stride, int rows, int width, const float *norm_w,
-                         float eps, int8_t *q, long plane, float *scale, hipStream_t stream) {
+                         float eps, int8_t *q, float *scale, hipStream_t stream) {
     if (!x || !q || !scale || rows <= 0 || width <= 0) return kErrArgs;
     QuantSeg a;
     a.x = x;
@@ -182,7 +185,6 @@ int quantize_activations(const float *x, long x_stride, int rows, int width, con
     a.norm_w = norm_w;
     a.eps = eps;
     a.q = q;
-    a.plane = plane;
     a.scale = scale;
     return quantize_segments(a, QuantSeg{}, stream);
 }
@@ -191,16 +193,27 @@ int quantize_activations(const float *x, long x_stride, int rows, int width, con
 // GEMM
 // ---------------------------------------------------------------------------
 
-// 16 packed nibbles (stored q + 8, column 2j low) -> 8 int8 values q.
+// 8 packed nibbles (stored q + 8, column 2j low) -> 8 int8 values in column
+// order, q or (TIMES16, two instructions less) 16 q: the nibble in the high
+// half of its byte with the offset taken off by an xor.
+template <bool TIMES16 = false>
 __device__ __forceinline__ void unpack_q4_word(unsigned w, unsigned &out0, unsigned &out1) {
-    const unsigned lo = w & 0x0F0F0F0Fu;         // even columns
-    const unsigned hi = (w >> 4) & 0x0F0F0F0Fu;  // odd columns
+    unsigned lo, hi;  // even and odd columns
+    if constexpr (TIMES16) {
+        lo = ((w << 4) & 0xF0F0F0F0u) ^ 0x80808080u;
+        hi = (w & 0xF0F0F0F0u) ^ 0x80808080u;
+    } else {
+        lo = w & 0x0F0F0F0Fu;
+        hi = (w >> 4) & 0x0F0F0F0Fu;
+    }
     // bytes [lo0, hi0, lo1, hi1] and [lo2, hi2, lo3, hi3]
-    const unsigned a = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
-    const unsigned b = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
-    // stored u in [0, 15] -> u - 8 as int8: (u + 0x78) ^ 0x80, no carry between bytes
-    out0 = (a + 0x78787878u) ^ 0x80808080u;
-    out1 = (b + 0x78787878u) ^ 0x80808080u;
+    out0 = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
+    out1 = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
+    if constexpr (!TIMES16) {
+        // stored u in [0, 15] -> u - 8 as int8: (u + 0x78) ^ 0x80, no carry between bytes
+        out0 = (out0 + 0x78787878u) ^ 0x80808080u;
+        out1 = (out1 + 0x78787878u) ^ 0x80808080u;
+    }
 }
 
 __device__ __forceinline__ int find_task(const int *tile_start, int n, int tile) {
@@ -274,63 +287,50 @@ __device__ __forceinline__ bool map_tile(const QGemmLaunch &L, GemmTask &tk, int
     return true;
 }
 
-// LDS tiles hold one k slice per stage as rows of RB bytes (RB / 16 chunks of
-// 16 bytes): q8 slices are 128 wide and go straight from global memory into
-// LDS (global_load_lds_dwordx4, full 128-byte lines per row); q4 slices are
-// 64 wide and are unpacked in registers on the way.  Chunk c of row r lives
-// at chunk c ^ g(r):
-//   RB = 64:  g(r) = ((r >> 1) ^ (r >> 3)) & 3
-//   RB = 128: g(r) = (r ^ (r >> 3)) & 7
+// LDS tiles hold one k slice of 128 per stage, as stored: activation rows and
+// q8 weight rows of 128 bytes, q4 weight rows of 64 (unpacked as they are
+// read), in 16-byte chunks.  Chunk c of row r lives at chunk c ^ g(r):
+//   rows of 64 bytes:  g(r) = ((r >> 1) ^ (r >> 3)) & 3
+//   rows of 128 bytes: g(r) = (r ^ (r >> 3)) & 7
 // so that the MFMA fragment reads (32 consecutive rows, one chunk) and the
 // tile writes hit distinct banks whether the LDS serves 8 or 16 lanes of a
 // 128-bit access per cycle.
-// q8 slices are 128 k wide, so a DMA instruction covers 8 rows x 128 contiguous
-// bytes (on MI355X runs of 128 bytes stream ~6 TB/s, runs of 64 bytes ~4.2
-// TB/s; the 128-row tile's fill alone took 2300 clocks a 64-k share against
-// 2900).  The 128-row tile's two stages fill the LDS.
-template <int FMT, int BM> struct QgCfg {
-    static constexpr int kRB = FMT == kQ8 ? 128 : 64;
-};
-
 template <int RB>
-__device__ __forceinline__ int lds_off(int row, int chunk) {
-    if constexpr (RB == 64) return row * 64 + ((chunk ^ (((row >> 1) ^ (row >> 3)) & 3)) << 4);
-    else return row * 128 + ((chunk ^ ((row ^ (row >> 3)) & 7)) << 4);
+__device__ __forceinline__ int lds_swizzle(int row) {
+    if constexpr (RB == 64) return ((row >> 1) ^ (row >> 3)) & 3;
+    else return (row ^ (row >> 3)) & 7;
 }
+
+constexpr int kQgSlice = 128;  // k per stage
 
 // Tile shape of a BM-row tile (BM = 128 or kQgBMSmall = 32).  BM = 128: 8
 // waves (two per SIMD) in a 4 (token rows) x 2 (weight rows) grid, each wave
-// 32 x 128 = 1 x 4 blocks of 32 x 32 per limb (192 int32 accumulators);
-// BM = 32: 4 waves side by side, each 32 x 64 = 1 x 2 blocks.  A stage holds
-// the three limb tiles of A and the weight tile.  q8 DMA: blocks of 1 KB
-// (1024 / kRB rows), wave w taking A blocks w, w + kWaves, ... (waves may
-// issue one more than others when the count does not divide), B blocks
-// likewise.
+// 32 x 128 = 4 blocks of 32 x 32 per limb (192 int32 accumulators);
+// BM = 32: 4 waves side by side, each 32 x 64 = 2 blocks.  A stage holds
+// the three limb tiles of A and the weight tile.  DMA: blocks of 1 KB, wave w
+// taking A blocks w, w + kWaves, ... (waves may issue one more than others
+// when the count does not divide), B blocks likewise.
 template <int FMT, int BM> struct QgShape {
-    static constexpr int kRB = QgCfg<FMT, BM>::kRB;
-    static constexpr int kRowsDma = 1024 / kRB;    // rows per DMA block
+    static constexpr int kRBB = FMT == kQ8 ? kQgSlice : kQgSlice / 2;  // bytes of a weight row
+    static constexpr int kRowsB = 1024 / kRBB;     // weight rows per DMA block
+    static constexpr int kRowsA = 8;
     static constexpr int kWaves = BM == 128 ? 8 : 4;
     static constexpr int kThreads = kWaves * kWave;
     static constexpr int kWM = BM / 32;            // waves along the token rows
     static constexpr int kWN = kWaves / kWM;       // waves along the weight rows
-    static constexpr int kMI = 1;
     static constexpr int kNF = kQgBW / 32 / kWN;   // 32-row weight blocks per wave
     static constexpr int kStages = FMT == kQ8 && BM == 32 ? 3 : 2;
-    static constexpr int kLdsA = kLimbs * BM * kRB;
-    static constexpr int kStage = (kLimbs * BM + kQgBW) * kRB;
+    static constexpr int kLdsA = kLimbs * BM * kQgSlice;
+    static constexpr int kStage = kLdsA + kQgBW * kRBB;
     static constexpr int kLds = kStages * kStage;
-    static constexpr int kRowBlocks = BM / kRowsDma;
+    static constexpr int kRowBlocks = BM / kRowsA;
     static constexpr int kAOffs = kRowBlocks > kWaves ? kRowBlocks / kWaves : 1;  // A row blocks per wave
     static constexpr int kABlocks = kLimbs * kRowBlocks;
-    static constexpr int kBBlocks = kQgBW / kRowsDma;
-    static constexpr int kBPer = kBBlocks / kWaves;
+    static constexpr int kBPer = kQgBW / kRowsB / kWaves;
     static constexpr int kAMax = (kABlocks + kWaves - 1) / kWaves, kAMin = kABlocks / kWaves;
     static constexpr int kDmaMax = kAMax + kBPer, kDmaMin = kAMin + kBPer;
-    // register path (q4): 16-byte A chunks and packed B chunks per thread and slice
-    static constexpr int kNA = (kLimbs * BM * 4 + kThreads - 1) / kThreads;
-    static constexpr int kNB = kQgBW * 2 / kThreads;
     static_assert(kWaves % kRowBlocks == 0 || kRowBlocks % kWaves == 0, "A row blocks of a wave");
-    static_assert(kBBlocks % kWaves == 0 && (kQgBW * 2) % kThreads == 0, "B split");
+    static_assert(kQgBW / kRowsB % kWaves == 0, "B split");
 };
 static_assert(QgShape<kQ8, kQgBM>::kLds <= 160 * 1024, "q8 128-row tile exceeds the LDS");
 static_assert(QgShape<kQ8, kQgBMSmall>::kLds <= 160 * 1024, "q8 32-row tile exceeds the LDS");
@@ -382,25 +382,23 @@ __device__ __forceinline__ float silu_times(float g, float u) {
 // a quarter, so the tile is bound by the weight stream instead of by padding.
 template <int FMT, bool DUAL, int BM>
 __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
-                             (BM == 128 || QgShape<FMT, BM>::kRB == 128) ? 1 : 2) void qgemm_kernel(
-    QGemmLaunch L) {
+                             (BM == 128 || FMT == kQ8) ? 1 : 2) void qgemm_kernel(QGemmLaunch L) {
     extern __shared__ __attribute__((aligned(16))) int8_t qg_lds[];
     using Sh = QgShape<FMT, BM>;
-    constexpr int kRB = Sh::kRB;
+    constexpr int kRBB = Sh::kRBB;
     constexpr int kStages = Sh::kStages;
     constexpr int kStage = Sh::kStage;
     constexpr int kLdsA = Sh::kLdsA;
-    constexpr int kMI = Sh::kMI, kNF = Sh::kNF;
-    constexpr bool kDma = FMT == kQ8;
+    constexpr int kNF = Sh::kNF;
     float *lds_scale = reinterpret_cast<float *>(qg_lds);  // after the products
     GemmTask tk;
     int m0, n0;
     if (!map_tile<DUAL, BM>(L, tk, m0, n0)) return;
 
-    constexpr int kThreads = Sh::kThreads;
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = tid >> 6;
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     // 128-row tiles: the two waves that share a SIMD (waves w and w + 4)
     // take 32-row blocks from different halves of the tile (wm and wm + 2)
     // and the same weight rows, so that in a tile of at most 64 token rows
@@ -411,305 +409,192 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
     // a wave whose 32 rows all lie past the task's end skips its products
     // (wave-uniform; it still issues its share of the copies and barriers)
     // (32-row tiles have one wave row: always live, no branch)
-    const bool live =
-        Sh::kWM == 1 || __builtin_amdgcn_readfirstlane(m0 + wm * (Sh::kMI * 32)) < tk.rows;
+    const bool live = Sh::kWM == 1 || __builtin_amdgcn_readfirstlane(m0 + wm * 32) < tk.rows;
 
-    // activation row of tile row r (past the task's end: row m0)
+    // activation row of tile row r (past the task's end: that of row m0)
     auto arow_of = [&](int r) {
         const int m = m0 + r < tk.rows ? m0 + r : m0;
-        return tk.a_rows ? tk.a_rows[m] : m;
+        return tk.a_rows ? tk.a_rows[m] : tk.a_row0 + m;
     };
-
-    // ---- per-thread global sources (fixed over k).  Rows past the task's end
-    // read row m0 (A) or weight row 0 (B): their outputs are never stored.
     const int w_ld = tk.w_ld ? tk.w_ld : tk.k;
     const long w_row_bytes = FMT == kQ8 ? w_ld : w_ld / 2;
-    const uint8_t *const w_gate = tk.w;
-    const uint8_t *const w_up = tk.w2;
-    // output / weight row held by LDS B row j: SwiGLU tiles give each wave
-    // its kNF / 2 gate blocks and then the matching up blocks (kNF = 4:
-    // blocks f = 0, 1 gate, 2, 3 up of a 128-row wave half; kNF = 2: block 0
-    // gate, 1 up of a 64-row wave quarter)
+    // the tile's first activation row block and weight row, in 64 bits: the
+    // offsets from there fit 32 (gathered rows are those of one routing call)
+    const int a_first = tk.a_rows ? 0 : (tk.a_row0 + m0) & ~7;
+    const int8_t *const a_base = tk.a + limb_at(a_first, 0, tk.a_width);
+    const uint8_t *const w_base = tk.w + n0 * w_row_bytes;
+    const uint8_t *const w2_base = DUAL ? tk.w2 + n0 * w_row_bytes : nullptr;
+    const long w_bytes = (tk.n_out - n0) * w_row_bytes;
+    // weight row from n0 held by LDS B row j: SwiGLU tiles give each wave its kNF / 2
+    // gate blocks and then the matching up blocks (kNF = 4: blocks f = 0, 1
+    // gate, 2, 3 up of a 128-row wave half; kNF = 2: block 0 gate, 1 up of a
+    // 64-row wave quarter)
     auto b_out = [&](int j, bool &up) -> int {
         if (!DUAL) {
             up = false;
-            return n0 + j;
+            return j;
         }
         constexpr int kHalf = kNF / 2;
         const int f = (j >> 5) % kNF;
         up = f >= kHalf;
-        return n0 + (j / (kNF * 32)) * (kHalf * 32) + (f % kHalf) * 32 + (j & 31);
-    };
-    auto b_row_src = [&](int j) -> const uint8_t * {
-        bool up;
-        const int out = b_out(j, up);
-        return (up ? w_up : w_gate) + (long)(out < tk.n_out ? out : 0) * w_row_bytes;
-    };
-    // limb planes at a fixed distance: the limb of an address is arithmetic,
-    // not a choice between pointers (which would put them in scratch memory)
-    const int8_t *const a_base = tk.a;
-    const long a_plane = tk.a_plane;
-    auto limb_base = [a_base, a_plane](int limb) -> const int8_t * {
-        return a_base + limb * a_plane;
-    };
-    auto a_row_src = [&](int limb, int r) -> const int8_t * {
-        return limb_base(limb) + (long)arow_of(r) * tk.a_stride;
+        return (j / (kNF * 32)) * (kHalf * 32) + (f % kHalf) * 32 + (j & 31);
     };
 
-    // DMA path (q8), blocks of R = 1024 / kRB rows = 1 KB: A block b holds
-    // limb b / kRowBlocks, rows (b % kRowBlocks) * R + l / (kRB / 16); wave w
-    // issues A blocks w, w + kWaves, ..., all in row block w % kRowBlocks,
-    // and B blocks (rows (w + kWaves q) * R + l / (kRB / 16)); lane l fills
-    // LDS row (block row 0 + l / (kRB / 16)), physical chunk l % (kRB / 16),
-    // so it loads the logical chunk (l % (kRB / 16)) ^ g(row).  The limbs
-    // share a lane's A rows.
-    constexpr int kCh = kRB / 16;
-    const int lr = lane / kCh, lc = lane % kCh;
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    auto swz = [](int r) { return kRB == 64 ? (((r >> 1) ^ (r >> 3)) & 3) : ((r ^ (r >> 3)) & 7); };
-    // byte offsets of this lane's A rows; past the task's end outside the
-    // buffer (read as zeros)
+    // DMA blocks of 1 KB: A block b holds limb b / kRowBlocks of the 8 tile
+    // rows 8 (b % kRowBlocks) ..; wave w issues A blocks w, w + kWaves, ...
+    // and B blocks likewise (kRowsB weight rows each).  Lane l fills the
+    // block's 16 bytes at 16 l: LDS row l / chunks, physical chunk l % chunks,
+    // so it loads the logical chunk (l % chunks) ^ g(row).  The limbs share a
+    // lane's A rows.  Byte offsets of this lane's A rows; past the task's end
+    // outside the buffer (read as zeros):
     constexpr long kABytes = 0xF0000000L;
+    const int alr = lane >> 3, alc = lane & 7;
     unsigned a_off[Sh::kAOffs];
-    // register path (q4, 64-byte rows): kNA A chunks and kNB packed B chunks
-    constexpr int kNA = Sh::kNA, kNB = Sh::kNB;
-    const int8_t *a_src[kNA];
-    int a_dst[kNA];
-    const uint8_t *b_src[kNB];
-    int b_dst[kNB];
-    u32x4 ra[kNA], rb[kNB];
-    if constexpr (kDma) {
 #pragma unroll
-        for (int h = 0; h < Sh::kAOffs; ++h) {
-            const int r = ((wave + Sh::kWaves * h) % Sh::kRowBlocks) * Sh::kRowsDma + lr;
-            a_off[h] = m0 + r < tk.rows ? (unsigned)(arow_of(r) * tk.a_stride) : (unsigned)kABytes;
-        }
-    } else {
-#pragma unroll
-        for (int q = 0; q < kNA; ++q) {
-            const int c = min(tid + kThreads * q, kLimbs * BM * 4 - 1);
-            const int limb = c / (4 * BM), r = (c >> 2) & (BM - 1), kc = c & 3;
-            a_src[q] = a_row_src(limb, r) + kc * 16;
-            a_dst[q] = limb * (BM * kRB) + lds_off<kRB>(r, kc);
-        }
-#pragma unroll
-        for (int q = 0; q < kNB; ++q) {
-            const int c = tid + kThreads * q;
-            const int j = c >> 1, part = c & 1;  // 32 packed columns per part
-            b_src[q] = b_row_src(j) + part * 16;
-            b_dst[q] = (j << 1) | part;
-        }
+    for (int h = 0; h < Sh::kAOffs; ++h) {
+        const int r = ((wave + Sh::kWaves * h) % Sh::kRowBlocks) * Sh::kRowsA + alr;
+        a_off[h] = m0 + r < tk.rows ? (unsigned)limb_at(arow_of(r) - a_first, 0, tk.a_width)
+                                    : (unsigned)kABytes;
     }
-
     // one k slice into LDS stage buf (kDmaMin or kDmaMax DMA instructions per
     // wave).  Buffer loads: with a flat LDS DMA in flight the compiler makes
     // every wait for an LDS read a wait for all of them.  Weight rows past
     // the task's last are out of the buffer's range and arrive as zeros.
-    auto issue_dma = [&](int k0, int buf) {
+    auto issue_dma = [&](int ks, int buf) {
         __attribute__((address_space(3))) int8_t *stage =
             (__attribute__((address_space(3))) int8_t *)(qg_lds + buf * kStage);
-        constexpr int kRowBlocks = Sh::kRowBlocks;
+        const int k0 = ks * kQgSlice;
 #pragma unroll
         for (int h = 0; h < Sh::kAMax; ++h) {
             const int b = wave_u + Sh::kWaves * h;  // A block
             if (h >= Sh::kAMin && b >= Sh::kABlocks) break;  // wave-uniform
-            const int limb = b / kRowBlocks, rb = b % kRowBlocks;
-            const int chunk = lc ^ swz(rb * Sh::kRowsDma + lr);
-            // a reduction that ends inside the slice: zeros past it
-            const bool past = k0 + kRB > tk.k && k0 + chunk * 16 >= tk.k;
-            dma16(buffer_of(limb_base(limb), kABytes),
-                  past ? (unsigned)kABytes : a_off[h % Sh::kAOffs] + (unsigned)(chunk * 16), k0,
-                  stage + b * 1024);
+            const int chunk = alc ^ lds_swizzle<kQgSlice>(b % Sh::kRowBlocks * Sh::kRowsA + alr);
+            // a reduction that ends inside the slice: zeros past it (whatever
+            // the weights hold there)
+            const bool past = k0 + kQgSlice > tk.k && k0 + chunk * 16 >= tk.k;
+            dma16(buffer_of(a_base, kABytes),
+                  past ? (unsigned)kABytes : a_off[h % Sh::kAOffs] + (unsigned)(chunk * 16),
+                  ks * kLimbBlock + b / Sh::kRowBlocks * 1024, stage + b * 1024);
         }
+        constexpr int kCh = kRBB / 16;
 #pragma unroll
         for (int q = 0; q < Sh::kBPer; ++q) {
             const int bb = wave_u + Sh::kWaves * q;
-            const int j = bb * Sh::kRowsDma + lr;  // B row of this lane
-            bool up;
-            (void)b_out(bb * Sh::kRowsDma, up);  // a block's rows are of one matrix
-            bool u;
-            dma16(buffer_of(up ? w_up : w_gate, tk.n_out * w_row_bytes),
-                  (unsigned)(b_out(j, u) * w_row_bytes) + (unsigned)((lc ^ swz(j)) * 16), k0,
+            const int j = bb * Sh::kRowsB + lane / kCh;  // B row of this lane
+            bool up, u;
+            (void)b_out(bb * Sh::kRowsB, up);  // a block's rows are of one matrix
+            const int chunk = (lane % kCh) ^ lds_swizzle<kRBB>(j);
+            dma16(buffer_of(up ? w2_base : w_base, w_bytes),
+                  (unsigned)(b_out(j, u) * w_row_bytes) + (unsigned)(chunk * 16), ks * kRBB,
                   stage + kLdsA + bb * 1024);
         }
     };
-    auto fetch = [&](int k0) {
-#pragma unroll
-        for (int q = 0; q < kNA; ++q) ra[q] = load_global16(a_src[q] + k0);
-#pragma unroll
-        for (int q = 0; q < kNB; ++q) rb[q] = load_global16(b_src[q] + k0 / 2);
-    };
-    auto stash = [&](int buf) {
-        int8_t *a = qg_lds + buf * kStage;
-#pragma unroll
-        for (int q = 0; q < kNA; ++q) *reinterpret_cast<u32x4 *>(a + a_dst[q]) = ra[q];
-        int8_t *b = a + kLdsA;
-#pragma unroll
-        for (int q = 0; q < kNB; ++q) {
-            const int j = b_dst[q] >> 1, part = b_dst[q] & 1;
-            unsigned v[8];
-            unpack_q4_word(rb[q].x, v[0], v[1]);
-            unpack_q4_word(rb[q].y, v[2], v[3]);
-            unpack_q4_word(rb[q].z, v[4], v[5]);
-            unpack_q4_word(rb[q].w, v[6], v[7]);
-            *reinterpret_cast<u32x4 *>(b + lds_off<kRB>(j, 2 * part)) =
-                u32x4{v[0], v[1], v[2], v[3]};
-            *reinterpret_cast<u32x4 *>(b + lds_off<kRB>(j, 2 * part + 1)) =
-                u32x4{v[4], v[5], v[6], v[7]};
-        }
-    };
 
-    i32x16 acc[kLimbs][kMI][kNF];  // [limb][row block][weight-row block]
+    i32x16 acc[kLimbs][kNF];  // [limb][weight-row block]
 #pragma unroll
     for (int a = 0; a < kLimbs; ++a)
 #pragma unroll
-        for (int i = 0; i < kMI; ++i)
+        for (int f = 0; f < kNF; ++f)
 #pragma unroll
-            for (int f = 0; f < kNF; ++f)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[a][i][f][r] = 0;
+            for (int r = 0; r < 16; ++r) acc[a][f][r] = 0;
 
+    // Fragments of step st (32 columns): lane half h takes 16 of them, q8
+    // chunk 2 st + h of both operands; q4 columns 64 (st / 2) + 32 h + 16
+    // (st % 2) .., so that a half's packed bytes of two steps are one chunk.
+    // LDS byte of this lane's first fragments: steps and blocks differ from
+    // it by an xor of the chunk bits (lds_swizzle; 32 rows on flip the top
+    // bit of a 128-byte row's swizzle) and by constants, computed where used:
+    // kept over the loop they would spill
     const int frow = lane & 31;
     const int half = lane >> 5;
-    // two 32-wide k steps: all fragments are read before the first MFMA so
-    // the LDS latency overlaps the MFMAs
-    auto compute_pair = [&](int buf, int ksub0) {
-        const int8_t *a0 = qg_lds + buf * kStage;
-        const int8_t *bb = a0 + kLdsA;
-        i32x4 fa[2][kLimbs][kMI], fb[2][kNF];
+    const int arow_lds = wm * 32 + frow, brow_lds = wn * (kNF * 32) + frow;
+    const int a_frag =
+        arow_lds * kQgSlice + (((FMT == kQ8 ? half : 2 * half) ^ lds_swizzle<kQgSlice>(arow_lds)) << 4);
+    const int b_frag = kLdsA + brow_lds * kRBB + ((half ^ lds_swizzle<kRBB>(brow_lds)) << 4);
+    using BRaw = typename std::conditional<FMT == kQ8, i32x4, u32x2>::type;
+    // Slices ks + 1 .. ks + kStages - 1 stream into LDS while slice ks is
+    // multiplied.  A wave's DMA completes in order, its kDmaMax or kDmaMin
+    // instructions per slice, so a slice has landed when at most that many for
+    // each later slice in flight remain; the barrier after the wait makes
+    // every wave's part visible and frees the stage of the slice before it.
+    // (A bare barrier: __syncthreads() would also wait for the loads of the
+    // fence it implies.)
+    static_assert(kStages == 2 || kStages == 3, "waits below");
+    const bool more = Sh::kDmaMax == Sh::kDmaMin || wave_u + Sh::kWaves * Sh::kAMin < Sh::kABlocks;
+    const int nk = (tk.k + kQgSlice - 1) / kQgSlice;
+    // slice ks has landed for every wave, and the stage of slice ks - 1 is
+    // free: it takes slice ks + kStages - 1
+    auto next_slice = [&](int ks) {
+        if (kStages == 3 && ks + 1 < nk) {
+            if (more) wait_vmcnt<Sh::kDmaMax>();
+            else wait_vmcnt<Sh::kDmaMin>();
+        } else {
+            wait_vmcnt<0>();
+        }
+        __builtin_amdgcn_s_barrier();
+        if (ks + kStages - 1 < nk) issue_dma(ks + kStages - 1, (ks + kStages - 1) % kStages);
+    };
+    // Fragments are read ahead of their products, the weights by two blocks
+    // and the activations by a step.  The sched_barriers keep the order: left
+    // to itself the compiler reads a block, waits for it and multiplies it,
+    // because the accumulators leave it few registers.  (Reading ahead across
+    // slices too, the barrier two blocks before a slice's end: the T = 2048 q8
+    // MoE layer 568 against 557 us.)
+    constexpr int kSteps = kQgSlice / 32, kBlocks = kSteps * kNF;
+    static_assert(kBlocks % 4 == 0 && kSteps == 4, "register rings, chunk bits");
+    i32x4 fa[2][kLimbs];
+    BRaw fb[4];
+    auto read_a = [&](int base, int st, int a) {
+        const int bits = FMT == kQ8 ? st << 5 : ((st & 1) << 4) | ((st >> 1) << 6);
+        fa[st & 1][a] = *reinterpret_cast<const i32x4 *>(qg_lds + ((base + a_frag) ^ bits) +
+                                                         a * (BM * kQgSlice));
+    };
+    auto read_b = [&](int base, int i) {
+        const int st = i / kNF, f = i % kNF;
+        const int bits = FMT == kQ8 ? (st << 5) ^ ((f & 1) << 6) : ((st >> 1) << 5) | ((st & 1) << 3);
+        fb[i % 4] = *reinterpret_cast<const BRaw *>(qg_lds + ((base + b_frag) ^ bits) + f * 32 * kRBB);
+    };
+    auto weights = [&](const BRaw &d) -> i32x4 {
+        if constexpr (FMT == kQ8) {
+            return d;
+        } else {
+            unsigned o0, o1, o2, o3;
+            unpack_q4_word<true>(d.x, o0, o1);
+            unpack_q4_word<true>(d.y, o2, o3);
+            return i32x4{(int)o0, (int)o1, (int)o2, (int)o3};
+        }
+    };
+    for (int st = 0; st < kStages - 1 && st < nk; ++st) issue_dma(st, st);
+    next_slice(0);
+    if (live) {
+        int base = 0;
+        for (int ks = 0; ks < nk; ++ks) {
+            if (ks) next_slice(ks);
+            asm("" : "+s"(base));  // (see a_frag)
 #pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-            const int chunk = (ksub0 + s2) * 2 + half;
+            for (int a = 0; a < kLimbs; ++a) read_a(base, 0, a);
+            read_b(base, 0);
+            read_b(base, 1);
 #pragma unroll
-            for (int i = 0; i < kMI; ++i) {
-                const int row = wm * (kMI * 32) + i * 32 + frow;
+            for (int i = 0; i < kBlocks; ++i) {
+                const int st = i / kNF, f = i % kNF;
+                if (i + 2 < kBlocks) read_b(base, i + 2);
+                if (st + 1 < kSteps) {
+                    constexpr int per = (kLimbs + kNF - 1) / kNF;
+#pragma unroll
+                    for (int a = f * per; a < (f + 1) * per && a < kLimbs; ++a) read_a(base, st + 1, a);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                const i32x4 w = weights(fb[i % 4]);
 #pragma unroll
                 for (int a = 0; a < kLimbs; ++a)
-                    fa[s2][a][i] = *reinterpret_cast<const i32x4 *>(a0 + a * (BM * kRB) +
-                                                                    lds_off<kRB>(row, chunk));
+                    acc[a][f] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[st & 1][a], w, acc[a][f], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
             }
-#pragma unroll
-            for (int f = 0; f < kNF; ++f) {
-                const int row = wn * (kNF * 32) + f * 32 + frow;
-                fb[s2][f] = *reinterpret_cast<const i32x4 *>(bb + lds_off<kRB>(row, chunk));
-            }
-        }
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-            for (int i = 0; i < kMI; ++i)
-#pragma unroll
-                for (int f = 0; f < kNF; ++f)
-#pragma unroll
-                    for (int a = 0; a < kLimbs; ++a)
-                        acc[a][i][f] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
-                            fa[s2][a][i], fb[s2][f], acc[a][i][f], 0, 0, 0);
-    };
-
-    // LDS byte of this lane's first A / B fragment.  Steps and blocks differ
-    // from it by an xor of bits 5 and 6 (lds_off: 16-byte chunk 2 st + half,
-    // swizzled by the row; 32 rows on flips the swizzle's top bit) and by
-    // constants, computed where used: kept over the loop they would spill
-    const int a_frag = lds_off<kRB>(wm * (kMI * 32) + frow, half);
-    const int b_frag = kLdsA + lds_off<kRB>(wn * (kNF * 32) + frow, half);
-    if constexpr (kDma) {
-        // Slices ks + 1 .. ks + kStages - 1 stream into LDS while slice ks is
-        // multiplied.  A wave's DMA completes in order, its kDmaMax or
-        // kDmaMin instructions per slice, so a slice has landed when at most
-        // that many for each later slice in flight remain; the barrier after
-        // the wait makes every wave's part visible and frees the stage of the
-        // slice before it.  (A bare barrier: __syncthreads() would also wait
-        // for the loads of the fence it implies.)
-        static_assert(kStages == 2 || kStages == 3, "waits below");
-        const bool more = Sh::kDmaMax == Sh::kDmaMin || wave_u + Sh::kWaves * Sh::kAMin < Sh::kABlocks;
-        const int nk = (tk.k + kRB - 1) / kRB;
-        // slice ks has landed for every wave, and the stage of slice ks - 1 is
-        // free: it takes slice ks + kStages - 1
-        auto next_slice = [&](int ks) {
-            if (kStages == 3 && ks + 1 < nk) {
-                if (more) wait_vmcnt<Sh::kDmaMax>();
-                else wait_vmcnt<Sh::kDmaMin>();
-            } else {
-                wait_vmcnt<0>();
-            }
-            __builtin_amdgcn_s_barrier();
-            if (ks + kStages - 1 < nk) issue_dma((ks + kStages - 1) * kRB, (ks + kStages - 1) % kStages);
-        };
-        // Fragments are read ahead of their products, the weights by two
-        // blocks and the activations by a step.  The sched_barriers keep the
-        // order: left to itself the compiler reads a block, waits for it and
-        // multiplies it, because the accumulators leave it few registers.
-        // (Reading ahead across slices too, the barrier two blocks before a
-        // slice's end: the T = 2048 q8 MoE layer 568 against 557 us.)  T = 2048 q8 MoE gate / up
-        // 350 -> 282 us with 128-wide slices, buffer DMA and this order.
-        constexpr int kSteps = kRB / 32, kBlocks = kSteps * kNF;
-        static_assert(kBlocks % 4 == 0 && kSteps % 2 == 0, "register rings");
-        i32x4 fa[2][kLimbs], fb[4];
-        auto read_a = [&](int base, int st, int a) {
-            fa[st & 1][a] = *reinterpret_cast<const i32x4 *>(qg_lds + ((base + a_frag) ^ (st % kSteps << 5)) +
-                                                             a * (BM * kRB));
-        };
-        auto read_b = [&](int base, int i) {
-            const int st = i / kNF, f = i % kNF;
-            fb[i % 4] = *reinterpret_cast<const i32x4 *>(
-                qg_lds + ((base + b_frag) ^ ((st << 5) ^ ((f & 1) << 6))) + f * 32 * kRB);
-        };
-        for (int st = 0; st < kStages - 1 && st < nk; ++st) issue_dma(st * kRB, st);
-        next_slice(0);
-        if (live) {
-            int base = 0;
-#pragma unroll
-            for (int a = 0; a < kLimbs; ++a) read_a(0, 0, a);
-            read_b(0, 0);
-            read_b(0, 1);
-            for (int ks = 0; ks < nk; ++ks) {
-                asm("" : "+s"(base));  // (see a_frag)
-                const int next = (ks + 1) % kStages * kStage;
-                if (ks) {
-                    next_slice(ks);
-#pragma unroll
-                    for (int a = 0; a < kLimbs; ++a) read_a(base, 0, a);
-                    read_b(base, 0);
-                    read_b(base, 1);
-                }
-#pragma unroll
-                for (int i = 0; i < kBlocks; ++i) {
-                    const int st = i / kNF, f = i % kNF;
-                    if (i + 2 < kBlocks) {
-                        read_b(base, i + 2);
-                    }
-                    if (st + 1 < kSteps) {
-                        constexpr int per = (kLimbs + kNF - 1) / kNF;
-#pragma unroll
-                        for (int a = f * per; a < (f + 1) * per && a < kLimbs; ++a) read_a(base, st + 1, a);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int a = 0; a < kLimbs; ++a)
-                        acc[a][0][f] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[st & 1][a], fb[i % 4],
-                                                                             acc[a][0][f], 0, 0, 0);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                base = next;
-            }
-        } else {
-            for (int ks = 1; ks < nk; ++ks) next_slice(ks);
+            base = (ks + 1) % kStages * kStage;
         }
     } else {
-        // two buffers: slice ks + 2 is in registers while slice ks is multiplied
-        const int nk = tk.k / kRB;
-        fetch(0);
-        stash(0);
-        if (nk > 1) fetch(kRB);
-        __syncthreads();
-        for (int ks = 0; ks < nk; ++ks) {
-            if (live) compute_pair(ks & 1, 0);
-            if (ks + 1 < nk) {
-                stash((ks + 1) & 1);
-                if (ks + 2 < nk) fetch((ks + 2) * kRB);
-            }
-            __syncthreads();
-        }
+        for (int ks = 1; ks < nk; ++ks) next_slice(ks);
     }
 
     // ---- epilogue, without a branch: stores and residual loads go through
@@ -725,7 +610,7 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
     const auto s_buf = buffer_of(tk.s, (long)tk.n_out * 4);
     const auto s2_buf = buffer_of(DUAL ? tk.s2 : tk.s, (long)tk.n_out * 4);
     const auto y_buf = buffer_of(tk.y + (long)m0 * tk.y_stride, (long)rows_here * tk.y_stride * 4);
-    const int lane_row = wm * (kMI * 32) + half * 4;  // + 8 (r / 4) + r % 4: row of result register r
+    const int lane_row = wm * 32 + half * 4;  // + 8 (r / 4) + r % 4: row of result register r
 #pragma unroll
     for (int f = 0; f < kF; ++f) {
         const int n = n0 + wn * kF * 32 + f * 32 + frow;
@@ -738,10 +623,12 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
     __syncthreads();
     if (tid < BM) lds_scale[tid] = tid < rows_here ? tk.a_scale[arow_of(tid)] : 0.0f;
     __syncthreads();
-    // 65536 hi + 256 mid + lo of one result register (the int32 sums are exact)
+    // 65536 hi + 256 mid + lo of one result register (the int32 sums are exact;
+    // q4 ones are 16 times the products')
     auto limb_sum = [&](int f, int r) -> float {
-        return fmaf((float)acc[0][0][f][r], 65536.0f,
-                    fmaf((float)acc[1][0][f][r], 256.0f, (float)acc[2][0][f][r]));
+        constexpr int kShift = FMT == kQ4 ? 4 : 0;
+        return fmaf((float)(acc[0][f][r] >> kShift), 65536.0f,
+                    fmaf((float)(acc[1][f][r] >> kShift), 256.0f, (float)(acc[2][f][r] >> kShift)));
     };
     auto epilogue = [&](auto with_resid) {
         constexpr bool kResid = decltype(with_resid)::value;
@@ -807,8 +694,6 @@ template <int FMT, int MB> struct QsShape {
     static_assert((kStages - 1) * kLoads <= 63, "vmcnt range");
 };
 
-typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-
 template <int FMT, bool DUAL, int MB>
 __global__ __launch_bounds__(256, 2) void qgemm_stream_kernel(QGemmLaunch L) {
     using Sh = QsShape<FMT, MB>;
@@ -832,8 +717,8 @@ __global__ __launch_bounds__(256, 2) void qgemm_stream_kernel(QGemmLaunch L) {
     for (int i = 0; i < MB; ++i) {
         const int m = m0 + 16 * i + l16;
         const int mm = m < tk.rows ? m : m0;
-        const int arow = tk.a_rows ? tk.a_rows[mm] : mm;
-        a_src[i] = tk.a + (long)arow * tk.a_stride + 16 * kq;
+        const int arow = tk.a_rows ? tk.a_rows[mm] : tk.a_row0 + mm;
+        a_src[i] = tk.a + limb_at(arow, 0, tk.a_width) + 16 * kq;
     }
     // weight row of LDS row j (0..63) of this wave: SwiGLU tiles give a wave
     // 32 gate rows (LDS rows 0..31) and the matching 32 up rows (32..63)
@@ -885,7 +770,7 @@ __global__ __launch_bounds__(256, 2) void qgemm_stream_kernel(QGemmLaunch L) {
 #pragma unroll
                 for (int i = 0; i < MB; ++i) {
                     const u32x4 v =
-                        load_global16(a_src[i] + a * tk.a_plane + (long)slice * 64);
+                        load_global16(a_src[i] + (slice >> 1) * kLimbBlock + a * 1024 + (slice & 1) * 64);
                     ra[st][h][a][i] = i32x4{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
                 }
         }
@@ -968,7 +853,7 @@ __global__ __launch_bounds__(256, 2) void qgemm_stream_kernel(QGemmLaunch L) {
         for (int r = 0; r < 4; ++r) {
             const int m = m0 + 16 * i + 4 * kq + r;
             const int mm = m < tk.rows ? m : m0;
-            sx[i][r] = load_global_f32(tk.a_scale + (tk.a_rows ? tk.a_rows[mm] : mm));
+            sx[i][r] = load_global_f32(tk.a_scale + (tk.a_rows ? tk.a_rows[mm] : tk.a_row0 + mm));
         }
     __builtin_amdgcn_s_waitcnt(0);
     auto limb_sum = [&](int i, int f, int r) -> float {
@@ -1101,9 +986,8 @@ static int host_tiles(bool dual, int rows, int n_out, int bm) {
 
 int qgemm_single(int fmt, bool dual, const GemmTask &task, hipStream_t stream) {
     if (!qgemm_shape_ok(fmt, task.k) || task.rows <= 0 || task.n_out <= 0 || !task.w ||
-        !task.s || !task.a || task.a_plane < (long)task.rows * task.a_stride || !task.a_scale ||
-        !task.y ||
-        (dual && (!task.w2 || !task.s2)) || task.a_stride % 16)
+        !task.s || !task.a || task.a_width < task.k || !task.a_scale || !task.y ||
+        (dual && (!task.w2 || !task.s2)))
         return kErrArgs;
     QGemmLaunch L;
     L.single = task;
@@ -1121,10 +1005,10 @@ struct MoeScheduleParams {
     int bm;  // token rows per tile of the launches that read the tables
 };
 
-// Tasks of the shared down projection: 2 k halves when its width is twice
-// inter and a second output exists, else 1.
+// Tasks of the shared down projection: 2 k halves where they can be and a
+// second output exists, else 1.
 __host__ __device__ inline int moe_shared_down_parts(const MoeGemmParams &p) {
-    return p.has_shared && p.shared_out2 && p.shared_width == 2 * p.inter ? 2 : 1;
+    return p.has_shared && p.shared_out2 && moe_shared_splits(p.inter, p.shared_width) ? 2 : 1;
 }
 
 // With L (routing in the same workgroup) the route tables and the expert
@@ -1156,9 +1040,8 @@ __device__ __forceinline__ void moe_schedule_body(const MoeScheduleParams &sp,
         a.n_out = p.inter;
         a.k = p.hidden;
         a.a = p.xq;
-        a.a_plane = p.xq_plane;
         a.a_scale = p.xq_scale;
-        a.a_stride = p.hidden;
+        a.a_width = p.hidden;
         a.a_rows = p.list_rows + off;
         a.y = p.expert_hidden + (long)off * p.inter;
         a.y_stride = p.inter;
@@ -1170,10 +1053,10 @@ __device__ __forceinline__ void moe_schedule_body(const MoeScheduleParams &sp,
         b.rows = cnt;
         b.n_out = p.hidden;
         b.k = p.inter;
-        b.a = p.hq + (long)off * p.inter;
-        b.a_plane = p.hq_plane;
-        b.a_scale = p.hq_scale + off;
-        b.a_stride = p.inter;
+        b.a = p.hq;
+        b.a_scale = p.hq_scale;
+        b.a_width = p.inter;
+        b.a_row0 = off;
         b.y = p.expert_out + (long)off * p.hidden;
         b.y_stride = p.hidden;
         t1[u] = b;
@@ -1193,9 +1076,8 @@ __device__ __forceinline__ void moe_schedule_body(const MoeScheduleParams &sp,
             a.n_out = p.shared_width;
             a.k = p.hidden;
             a.a = p.xq;
-            a.a_plane = p.xq_plane;
-            a.a_scale = p.xq_scale;
-            a.a_stride = p.hidden;
+                a.a_scale = p.xq_scale;
+            a.a_width = p.hidden;
             a.y = p.shared_hidden;
             a.y_stride = p.shared_width;
             t0[nr] = a;
@@ -1213,10 +1095,9 @@ __device__ __forceinline__ void moe_schedule_body(const MoeScheduleParams &sp,
                 b.n_out = p.hidden;
                 b.k = kpart;
                 b.w_ld = p.shared_width;
-                b.a = p.sq + col;
-                b.a_plane = p.sq_plane;
+                b.a = p.sq + limb_at(0, (int)col, p.shared_width);
                 b.a_scale = p.sq_scale;
-                b.a_stride = p.shared_width;
+                b.a_width = p.shared_width;
                 b.y = i == 0 ? p.shared_out : p.shared_out2;
                 b.y_stride = p.hidden;
                 t1[nr + i] = b;
@@ -1319,7 +1200,6 @@ int moe_gemm(const MoeGemmParams &p, hipStream_t stream) {
     xs.norm_w = p.norm_w;
     xs.eps = p.eps;
     xs.q = p.xq;
-    xs.plane = p.xq_plane;
     xs.scale = p.xq_scale;
     if (!p.x || !p.xq || !p.xq_scale || !quant_seg_ok(xs))
         return kErrArgs;
@@ -1377,7 +1257,6 @@ int moe_gemm(const MoeGemmParams &p, hipStream_t stream) {
             hs.rows = entries;
             hs.width = p.inter;
             hs.q = p.hq;
-            hs.plane = p.hq_plane;
             hs.scale = p.hq_scale;
             if (p.has_shared) {
                 ss.x = p.shared_hidden;
@@ -1385,7 +1264,6 @@ int moe_gemm(const MoeGemmParams &p, hipStream_t stream) {
                 ss.rows = p.rows;
                 ss.width = p.shared_width;
                 ss.q = p.sq;
-                ss.plane = p.sq_plane;
                 ss.scale = p.sq_scale;
             }
             st = quantize_segments(hs, ss, stream);

@@ -139,14 +139,12 @@ struct MoonlightSession {
     float *shared_out2 = nullptr;  // second k half of the GEMM path's shared down
     float *moe_routed = nullptr;  // routed part of moonlight_test_moe
     // MFMA path for batches of >= kMoeGemmMinRows token rows
-    // quantised activations: three limb planes [3][max_batch][aq_width]
+    // quantised activations: limb blocks of [max_batch][aq_width]
     int8_t *aq = nullptr;
-    long aq_plane = 0;
     float *aq_scale = nullptr;
     int aq_width = 0;
-    // quantised expert hidden: three limb planes [3][max_batch*K][inter]
+    // quantised expert hidden: limb blocks of [max_batch*K][inter]
     int8_t *hq = nullptr;
-    long hq_plane = 0;
     float *hq_scale = nullptr;
     GemmTask *gemm_tasks = nullptr;
     int *gemm_tile_start = nullptr;
@@ -936,7 +934,7 @@ int gemm_rows(MoonlightSession *s, const Matrix &m, const Matrix *up, const floa
               int in_w, int out_w, float *y, const float *norm_w, const float *resid) {
     hipStream_t st = stream_of(s);
     if (int e = quantize_activations(x, in_w, rows, in_w, norm_w, s->model->cfg.rms_norm_epsilon,
-                                     s->aq, s->aq_plane, s->aq_scale, st))
+                                     s->aq, s->aq_scale, st))
         return e;
     GemmTask t;
     t.w = m.w;
@@ -949,9 +947,8 @@ int gemm_rows(MoonlightSession *s, const Matrix &m, const Matrix *up, const floa
     t.n_out = out_w;
     t.k = in_w;
     t.a = s->aq;
-    t.a_plane = s->aq_plane;
     t.a_scale = s->aq_scale;
-    t.a_stride = in_w;
+    t.a_width = in_w;
     t.y = y;
     t.y_stride = out_w;
     t.resid = resid;
@@ -1269,9 +1266,9 @@ int experts(MoonlightSession *s, int layer, const float *x, int rows, const floa
     f.shared_hidden = s->shared_hidden;
     f.shared_out = s->shared_out;
     const bool gemm = moe_uses_gemm(s, layer, rows);
-    // the GEMM path runs a shared down projection twice inter wide as two k
-    // halves into shared_out and shared_out2 (moe_shared_down_parts)
-    const bool split_shared = gemm && f.shared_width == 2 * f.inter;
+    // the GEMM path runs such a shared down projection as two k halves into
+    // shared_out and shared_out2
+    const bool split_shared = gemm && moe_shared_splits(f.inter, f.shared_width);
     if (gemm) {
         MoeGemmParams g;
         g.rows = f.rows;
@@ -1305,10 +1302,8 @@ int experts(MoonlightSession *s, int layer, const float *x, int rows, const floa
         // the token-row quantisation is consumed by stage 0 before the shared
         // hidden is quantised into the same buffer
         g.xq = g.sq = s->aq;
-        g.xq_plane = g.sq_plane = s->aq_plane;
         g.xq_scale = g.sq_scale = s->aq_scale;
         g.hq = s->hq;
-        g.hq_plane = s->hq_plane;
         g.hq_scale = s->hq_scale;
         g.tasks = s->gemm_tasks;
         g.tile_start = s->gemm_tile_start;
@@ -1699,11 +1694,10 @@ extern "C" int moonlight_session_create(MoonlightSession **out, MoonlightModel *
         int aw = 0;
         for (int w : widths) aw = w > aw ? w : aw;
         s->aq_width = aw;
-        s->aq_plane = (long)(mb * (size_t)aw);
-        s->hq_plane = (long)(mb * K * (size_t)c.moe_intermediate_size);
-        gemm_ok = session_alloc(s, &s->aq, 3 * (size_t)s->aq_plane, error, error_size) &&
+        gemm_ok = session_alloc(s, &s->aq, (size_t)limb_bytes((long)mb, aw), error, error_size) &&
                   session_alloc(s, &s->aq_scale, mb, error, error_size) &&
-                  session_alloc(s, &s->hq, 3 * (size_t)s->hq_plane, error, error_size) &&
+                  session_alloc(s, &s->hq, (size_t)limb_bytes((long)(mb * K), c.moe_intermediate_size), error,
+                                error_size) &&
                   session_alloc(s, &s->hq_scale, mb * K, error, error_size) &&
                   session_alloc(s, &s->gemm_tasks, 2 * (size_t)kQgMaxTasks, error, error_size) &&
                   session_alloc(s, &s->gemm_tile_start, 2 * (size_t)(kQgMaxTasks + 1), error,
