@@ -7,6 +7,7 @@
 
 #include "gemv_impl.h"
 #include "moe.h"
+#include "qgemm.h"
 
 namespace mlh {
 
@@ -289,7 +290,8 @@ std::string gemv_kernel_name(int fmt, int O, int I, int rows, bool dual) {
     q.epilogue = dual ? kEpiSiluDual : q.epilogue;
     std::string mfma;
     q.x_stride = I;
-    if (gemv_mfma(q, nullptr, &mfma) || (!vector_first(q, vector_takes(q)) && gemv_batch(q, nullptr, &mfma)))
+    if (gemv_mfma(q, nullptr, &mfma) ||
+        (q.rows > 4 && !gemv_batch_fits(q) && gemv_tiles(q, nullptr, &mfma)) || (!vector_first(q, vector_takes(q)) && gemv_batch(q, nullptr, &mfma)))
         return mfma;
     const GemvPlan pl = plan_gemv(fmt, O, I, rows < kMaxGemvRows ? rows : kMaxGemvRows, dual);
     char buf[96];
@@ -315,6 +317,8 @@ int gemv(const GemvParams &p_in, hipStream_t stream) {
     if (gemv_mfma(p_in, stream))
         return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
     if (p_in.router_parts) return kErrArgs;
+    if (p_in.rows > 4 && !gemv_batch_fits(p_in) && gemv_tiles(p_in, stream))
+        return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
     const bool vector_ok = vector_takes(p_in);
     if (!vector_first(p_in, vector_ok) && gemv_batch(p_in, stream))
         return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;

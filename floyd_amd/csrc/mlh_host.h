@@ -54,6 +54,23 @@ struct GemvParams {
 };
 
 int gemv(const GemvParams &p, hipStream_t stream);
+
+// Whether a q8 / q4 projection of several token rows stays on the batch kernel
+// (gemv_batch.hip, one launch, x split in every workgroup) rather than
+// quantising its rows once for the GEMM tiles (qgemm.hip).  The batch kernel
+// takes 30 us per 1000 workgroups of 64 weight rows, 16 token rows and 2048
+// columns; the tiles take 28 us for 2048 columns, 50 for 4096 and 120 for 11264
+// until their tiles fill the CUs.  Measured on MI355X, batch against tiles: 3072
+// x 2048 at 256 rows 28.9 / 29.9 us, at 512 56.7 / 32.6; 11264 x 2048 at 64 rows
+// 29.3 / 31.6, at 128 56.7 / 32.1; 8000 x 4096 at 64 rows 36.7 / 56.0, at 300
+// 173 / 58; 2048 x 11264 at 256 rows 87 / 123, at 777 282 / 139.
+inline bool gemv_batch_fits(long weight_rows, int rows, int in_width) {
+    const long chunks = (in_width + 2047) / 2048;
+    return (weight_rows + 63) / 64 * ((rows + 15) / 16) * chunks <= 300 + 600 * chunks;
+}
+inline bool gemv_batch_fits(const GemvParams &p) {
+    return gemv_batch_fits((long)p.O * (p.epilogue == kEpiSiluDual ? 2 : 1), p.rows, p.I);
+}
 // Whether gemv() can write router logit partials for p (router fields
 // aside), and how many partials per expert it then writes.
 bool gemv_router_ok(const GemvParams &p);

@@ -25,6 +25,7 @@
 namespace mlh {
 
 constexpr int kQgBM = 128;  // token rows per tile
+constexpr int kQgBMMid = 64;
 constexpr int kQgBMSmall = 32;  // token rows per tile of few-row launches
 constexpr int kQgBW = 256;  // weight rows per tile
 constexpr int kQgBK = 64;   // k per pipeline stage
@@ -37,16 +38,20 @@ constexpr int kQgMaxTasks = 272;
 // piece where its rows follow each other (a probe of the tile's fill alone:
 // 1780 clocks a 64-k share from such pieces, 2300 from 128-byte runs of limb
 // planes, 2900 from 64-byte runs).
-constexpr int kLimbBlock = 3 * 8 * 128;
+constexpr int kLimbs = 3;
+template <int LIMBS = kLimbs>
 __host__ __device__ inline long limb_row_block(int width) {  // bytes per 8 rows
-    return (long)((width + 127) / 128) * kLimbBlock;
+    return (long)((width + 127) / 128) * (LIMBS * 1024);
 }
+template <int LIMBS = kLimbs>
 __host__ __device__ inline long limb_bytes(long rows, int width) {
-    return (rows + 7) / 8 * limb_row_block(width);
+    return (rows + 7) / 8 * limb_row_block<LIMBS>(width);
 }
 // Byte of limb 0 at (row, col); limb l is 1024 l further.
+template <int LIMBS = kLimbs>
 __host__ __device__ inline long limb_at(long row, int col, int width) {
-    return (row >> 3) * limb_row_block(width) + (col >> 7) * kLimbBlock + (row & 7) * 128 + (col & 127);
+    return (row >> 3) * limb_row_block<LIMBS>(width) + (col >> 7) * (LIMBS * 1024) + (row & 7) * 128 +
+           (col & 127);
 }
 
 // One independent product: rows x n_out outputs, reduction length k.
@@ -88,6 +93,13 @@ int quantize_activations(const float *x, long x_stride, int rows, int width, con
 // One dense task, e.g. a prefill projection.  Epilogue: plain or residual
 // (task.resid) or SwiGLU pair (dual, task.w2 = up).
 int qgemm_single(int fmt, bool dual, const GemmTask &task, hipStream_t stream);
+
+// gemv() of many token rows on the same tiles with four limbs (30 bits of the
+// row's largest value, as the other matrix-core GEMVs): quantises the rows
+// into the library's own scratch and multiplies.  False, launching nothing,
+// for shapes it does not take; with `name` set it launches nothing and stores
+// the kernel's template name.
+bool gemv_tiles(const GemvParams &p, hipStream_t stream, std::string *name = nullptr);
 
 // MoE prefill: builds the per-expert task tables from the device route tables
 // and runs both expert stages for all active experts plus the shared expert.

@@ -20,8 +20,14 @@
 // C[(r / 4) * 8 + (l / 32) * 4 + r % 4][l % 32].
 #include "qgemm.h"
 
+#include <algorithm>
+#include <cstdio>
 #include <cstdlib>
+#include <mutex>
+#include <string>
 #include <type_traits>
+
+#include "limb_split.h"
 
 namespace mlh {
 
@@ -29,7 +35,6 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kLimbs = 3;
 constexpr float kQuantMax = 4194304.0f;  // 2^22: |65536 * hi + 256 * mid + lo| bound
 
 bool qgemm_shape_ok(int fmt, int k) {
@@ -137,7 +142,7 @@ __device__ __forceinline__ void quantize_row(const QuantSeg &s, int row) {
         quant_limbs(t.y, inv, h1, m1, l1);
         quant_limbs(t.z, inv, h2, m2, l2);
         quant_limbs(t.w, inv, h3, m3, l3);
-        int8_t *at = qr + (i >> 7) * kLimbBlock + (i & 127);
+        int8_t *at = qr + (i >> 7) * (kLimbs * 1024) + (i & 127);
         *reinterpret_cast<unsigned *>(at) = pack_bytes(h0, h1, h2, h3);
         *reinterpret_cast<unsigned *>(at + 1024) = pack_bytes(m0, m1, m2, m3);
         *reinterpret_cast<unsigned *>(at + 2048) = pack_bytes(l0, l1, l2, l3);
@@ -303,29 +308,30 @@ __device__ __forceinline__ int lds_swizzle(int row) {
 
 constexpr int kQgSlice = 128;  // k per stage
 
-// Tile shape of a BM-row tile (BM = 128 or kQgBMSmall = 32).  BM = 128: 8
-// waves (two per SIMD) in a 4 (token rows) x 2 (weight rows) grid, each wave
-// 32 x 128 = 4 blocks of 32 x 32 per limb (192 int32 accumulators);
-// BM = 32: 4 waves side by side, each 32 x 64 = 2 blocks.  A stage holds
+// Tile shape of a BM-row tile (BM = 128, kQgBMMid = 64 or kQgBMSmall = 32).
+// BM = 128: 8 waves (two per SIMD) in a 4 (token rows) x 2 (weight rows) grid,
+// each wave 32 x 128 = 4 blocks of 32 x 32 per limb (192 int32 accumulators);
+// BM = 64: 8 waves in a 2 x 4 grid, each 32 x 64 = 2 blocks; BM = 32: 4 waves
+// side by side, each 32 x 64.  A stage holds
 // the three limb tiles of A and the weight tile.  DMA: blocks of 1 KB, wave w
 // taking A blocks w, w + kWaves, ... (waves may issue one more than others
 // when the count does not divide), B blocks likewise.
-template <int FMT, int BM> struct QgShape {
+template <int FMT, int BM, int LIMBS = kLimbs> struct QgShape {
     static constexpr int kRBB = FMT == kQ8 ? kQgSlice : kQgSlice / 2;  // bytes of a weight row
     static constexpr int kRowsB = 1024 / kRBB;     // weight rows per DMA block
     static constexpr int kRowsA = 8;
-    static constexpr int kWaves = BM == 128 ? 8 : 4;
+    static constexpr int kWaves = BM == 32 ? 4 : 8;
     static constexpr int kThreads = kWaves * kWave;
     static constexpr int kWM = BM / 32;            // waves along the token rows
     static constexpr int kWN = kWaves / kWM;       // waves along the weight rows
     static constexpr int kNF = kQgBW / 32 / kWN;   // 32-row weight blocks per wave
     static constexpr int kStages = FMT == kQ8 && BM == 32 ? 3 : 2;
-    static constexpr int kLdsA = kLimbs * BM * kQgSlice;
+    static constexpr int kLdsA = LIMBS * BM * kQgSlice;
     static constexpr int kStage = kLdsA + kQgBW * kRBB;
     static constexpr int kLds = kStages * kStage;
     static constexpr int kRowBlocks = BM / kRowsA;
     static constexpr int kAOffs = kRowBlocks > kWaves ? kRowBlocks / kWaves : 1;  // A row blocks per wave
-    static constexpr int kABlocks = kLimbs * kRowBlocks;
+    static constexpr int kABlocks = LIMBS * kRowBlocks;
     static constexpr int kBPer = kQgBW / kRowsB / kWaves;
     static constexpr int kAMax = (kABlocks + kWaves - 1) / kWaves, kAMin = kABlocks / kWaves;
     static constexpr int kDmaMax = kAMax + kBPer, kDmaMin = kAMin + kBPer;
@@ -333,6 +339,7 @@ template <int FMT, int BM> struct QgShape {
     static_assert(kQgBW / kRowsB % kWaves == 0, "B split");
 };
 static_assert(QgShape<kQ8, kQgBM>::kLds <= 160 * 1024, "q8 128-row tile exceeds the LDS");
+static_assert(QgShape<kQ8, kQgBMMid, 4>::kLds <= 160 * 1024, "q8 four-limb tile exceeds the LDS");
 static_assert(QgShape<kQ8, kQgBMSmall>::kLds <= 160 * 1024, "q8 32-row tile exceeds the LDS");
 static_assert(2 * QgShape<kQ4, kQgBMSmall>::kLds <= 160 * 1024, "two q4 32-row tiles per CU");
 
@@ -380,11 +387,11 @@ __device__ __forceinline__ float silu_times(float g, float u) {
 // Workgroup over a BM x 256 tile (QgShape).  The 32-row tile serves
 // batches whose experts hold few rows each: the MFMA work per weight byte is
 // a quarter, so the tile is bound by the weight stream instead of by padding.
-template <int FMT, bool DUAL, int BM>
-__global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
-                             (BM == 128 || FMT == kQ8) ? 1 : 2) void qgemm_kernel(QGemmLaunch L) {
+template <int FMT, bool DUAL, int BM, int LIMBS>
+__global__ __launch_bounds__((QgShape<FMT, BM, LIMBS>::kThreads),
+                             (BM != 32 || FMT == kQ8) ? 1 : 2) void qgemm_kernel(QGemmLaunch L) {
     extern __shared__ __attribute__((aligned(16))) int8_t qg_lds[];
-    using Sh = QgShape<FMT, BM>;
+    using Sh = QgShape<FMT, BM, LIMBS>;
     constexpr int kRBB = Sh::kRBB;
     constexpr int kStages = Sh::kStages;
     constexpr int kStage = Sh::kStage;
@@ -399,13 +406,14 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
     const int lane = tid & (kWave - 1);
     const int wave = tid >> 6;
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    // 128-row tiles: the two waves that share a SIMD (waves w and w + 4)
-    // take 32-row blocks from different halves of the tile (wm and wm + 2)
-    // and the same weight rows, so that in a tile of at most 64 token rows
-    // every SIMD still has one wave with products to run.
-    const int wm = Sh::kWM == 4 ? (wave & 1) | ((wave >> 2) << 1) : wave % Sh::kWM;
-    const int wn = Sh::kWM == 4 ? (wave >> 1) & 1 : wave / Sh::kWM;
-    static_assert(Sh::kWM == 1 || (Sh::kWM == 4 && Sh::kWN == 2), "wave grid");
+    // 8 waves: the two that share a SIMD (waves w and w + 4) take 32-row
+    // blocks from different halves of the tile and the same weight rows, so
+    // that in a tile whose second half is empty every SIMD still has one wave
+    // with products to run.
+    constexpr int kHalfM = Sh::kWM == 1 ? 1 : Sh::kWM / 2;  // row blocks of a half
+    const int wm = Sh::kWM == 1 ? 0 : wave % kHalfM + (wave >> 2) * kHalfM;
+    const int wn = Sh::kWM == 1 ? wave : (wave & 3) / kHalfM;
+    static_assert(Sh::kWM == 1 || Sh::kWM * Sh::kWN == 8, "wave grid");
     // a wave whose 32 rows all lie past the task's end skips its products
     // (wave-uniform; it still issues its share of the copies and barriers)
     // (32-row tiles have one wave row: always live, no branch)
@@ -421,7 +429,7 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
     // the tile's first activation row block and weight row, in 64 bits: the
     // offsets from there fit 32 (gathered rows are those of one routing call)
     const int a_first = tk.a_rows ? 0 : (tk.a_row0 + m0) & ~7;
-    const int8_t *const a_base = tk.a + limb_at(a_first, 0, tk.a_width);
+    const int8_t *const a_base = tk.a + limb_at<LIMBS>(a_first, 0, tk.a_width);
     const uint8_t *const w_base = tk.w + n0 * w_row_bytes;
     const uint8_t *const w2_base = DUAL ? tk.w2 + n0 * w_row_bytes : nullptr;
     const long w_bytes = (tk.n_out - n0) * w_row_bytes;
@@ -453,7 +461,7 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
 #pragma unroll
     for (int h = 0; h < Sh::kAOffs; ++h) {
         const int r = ((wave + Sh::kWaves * h) % Sh::kRowBlocks) * Sh::kRowsA + alr;
-        a_off[h] = m0 + r < tk.rows ? (unsigned)limb_at(arow_of(r) - a_first, 0, tk.a_width)
+        a_off[h] = m0 + r < tk.rows ? (unsigned)limb_at<LIMBS>(arow_of(r) - a_first, 0, tk.a_width)
                                     : (unsigned)kABytes;
     }
     // one k slice into LDS stage buf (kDmaMin or kDmaMax DMA instructions per
@@ -474,7 +482,7 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
             const bool past = k0 + kQgSlice > tk.k && k0 + chunk * 16 >= tk.k;
             dma16(buffer_of(a_base, kABytes),
                   past ? (unsigned)kABytes : a_off[h % Sh::kAOffs] + (unsigned)(chunk * 16),
-                  ks * kLimbBlock + b / Sh::kRowBlocks * 1024, stage + b * 1024);
+                  ks * (LIMBS * 1024) + b / Sh::kRowBlocks * 1024, stage + b * 1024);
         }
         constexpr int kCh = kRBB / 16;
 #pragma unroll
@@ -490,9 +498,9 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
         }
     };
 
-    i32x16 acc[kLimbs][kNF];  // [limb][weight-row block]
+    i32x16 acc[LIMBS][kNF];  // [limb][weight-row block]
 #pragma unroll
-    for (int a = 0; a < kLimbs; ++a)
+    for (int a = 0; a < LIMBS; ++a)
 #pragma unroll
         for (int f = 0; f < kNF; ++f)
 #pragma unroll
@@ -542,7 +550,7 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
     // MoE layer 568 against 557 us.)
     constexpr int kSteps = kQgSlice / 32, kBlocks = kSteps * kNF;
     static_assert(kBlocks % 4 == 0 && kSteps == 4, "register rings, chunk bits");
-    i32x4 fa[2][kLimbs];
+    i32x4 fa[2][LIMBS];
     BRaw fb[4];
     auto read_a = [&](int base, int st, int a) {
         const int bits = FMT == kQ8 ? st << 5 : ((st & 1) << 4) | ((st >> 1) << 6);
@@ -572,7 +580,7 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
             if (ks) next_slice(ks);
             asm("" : "+s"(base));  // (see a_frag)
 #pragma unroll
-            for (int a = 0; a < kLimbs; ++a) read_a(base, 0, a);
+            for (int a = 0; a < LIMBS; ++a) read_a(base, 0, a);
             read_b(base, 0);
             read_b(base, 1);
 #pragma unroll
@@ -580,14 +588,14 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
                 const int st = i / kNF, f = i % kNF;
                 if (i + 2 < kBlocks) read_b(base, i + 2);
                 if (st + 1 < kSteps) {
-                    constexpr int per = (kLimbs + kNF - 1) / kNF;
+                    constexpr int per = (LIMBS + kNF - 1) / kNF;
 #pragma unroll
-                    for (int a = f * per; a < (f + 1) * per && a < kLimbs; ++a) read_a(base, st + 1, a);
+                    for (int a = f * per; a < (f + 1) * per && a < LIMBS; ++a) read_a(base, st + 1, a);
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 const i32x4 w = weights(fb[i % 4]);
 #pragma unroll
-                for (int a = 0; a < kLimbs; ++a)
+                for (int a = 0; a < LIMBS; ++a)
                     acc[a][f] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[st & 1][a], w, acc[a][f], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -623,12 +631,17 @@ __global__ __launch_bounds__((QgShape<FMT, BM>::kThreads),
     __syncthreads();
     if (tid < BM) lds_scale[tid] = tid < rows_here ? tk.a_scale[arow_of(tid)] : 0.0f;
     __syncthreads();
-    // 65536 hi + 256 mid + lo of one result register (the int32 sums are exact;
-    // q4 ones are 16 times the products')
+    // the limbs' sum of one result register, 256 apart (the int32 sums are
+    // exact; q4 ones are 16 times the products')
     auto limb_sum = [&](int f, int r) -> float {
         constexpr int kShift = FMT == kQ4 ? 4 : 0;
-        return fmaf((float)(acc[0][f][r] >> kShift), 65536.0f,
-                    fmaf((float)(acc[1][f][r] >> kShift), 256.0f, (float)(acc[2][f][r] >> kShift)));
+        float v = (float)(acc[LIMBS - 1][f][r] >> kShift), unit = 1.0f;
+#pragma unroll
+        for (int a = LIMBS - 2; a >= 0; --a) {
+            unit *= 256.0f;
+            v = fmaf((float)(acc[a][f][r] >> kShift), unit, v);
+        }
+        return v;
     };
     auto epilogue = [&](auto with_resid) {
         constexpr bool kResid = decltype(with_resid)::value;
@@ -770,7 +783,7 @@ __global__ __launch_bounds__(256, 2) void qgemm_stream_kernel(QGemmLaunch L) {
 #pragma unroll
                 for (int i = 0; i < MB; ++i) {
                     const u32x4 v =
-                        load_global16(a_src[i] + (slice >> 1) * kLimbBlock + a * 1024 + (slice & 1) * 64);
+                        load_global16(a_src[i] + (slice >> 1) * (kLimbs * 1024) + a * 1024 + (slice & 1) * 64);
                     ra[st][h][a][i] = i32x4{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
                 }
         }
@@ -885,28 +898,28 @@ __global__ __launch_bounds__(256, 2) void qgemm_stream_kernel(QGemmLaunch L) {
         }
 }
 
-template <int FMT, bool DUAL, int BM>
+template <int FMT, bool DUAL, int BM, int LIMBS = kLimbs>
 static void launch_qgemm(const QGemmLaunch &L, int grid, hipStream_t stream) {
-    constexpr int kLds = QgShape<FMT, BM>::kLds;
+    using Sh = QgShape<FMT, BM, LIMBS>;
     static const bool attr = [] {
-        return hipFuncSetAttribute(reinterpret_cast<const void *>(&qgemm_kernel<FMT, DUAL, BM>),
+        return hipFuncSetAttribute(reinterpret_cast<const void *>(&qgemm_kernel<FMT, DUAL, BM, LIMBS>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   kLds) == hipSuccess;
+                                   Sh::kLds) == hipSuccess;
     }();
     (void)attr;
-    hipLaunchKernelGGL((qgemm_kernel<FMT, DUAL, BM>), dim3((unsigned)grid),
-                       dim3(QgShape<FMT, BM>::kThreads), kLds, stream, L);
+    hipLaunchKernelGGL((qgemm_kernel<FMT, DUAL, BM, LIMBS>), dim3((unsigned)grid), dim3(Sh::kThreads),
+                       Sh::kLds, stream, L);
 }
 
-template <int BM>
+template <int BM, int LIMBS = kLimbs>
 static void launch_qgemm_bm(int fmt, bool dual, const QGemmLaunch &L, int grid,
                             hipStream_t stream) {
     if (fmt == kQ8) {
-        if (dual) launch_qgemm<kQ8, true, BM>(L, grid, stream);
-        else launch_qgemm<kQ8, false, BM>(L, grid, stream);
+        if (dual) launch_qgemm<kQ8, true, BM, LIMBS>(L, grid, stream);
+        else launch_qgemm<kQ8, false, BM, LIMBS>(L, grid, stream);
     } else {
-        if (dual) launch_qgemm<kQ4, true, BM>(L, grid, stream);
-        else launch_qgemm<kQ4, false, BM>(L, grid, stream);
+        if (dual) launch_qgemm<kQ4, true, BM, LIMBS>(L, grid, stream);
+        else launch_qgemm<kQ4, false, BM, LIMBS>(L, grid, stream);
     }
 }
 
@@ -936,23 +949,31 @@ static void launch_stream_mb(int fmt, bool dual, const QGemmLaunch &L, int grid,
 }
 
 // Tile kinds: the weight-streaming tile with 16 token rows, the LDS tiles
-// with 32 or 128.
-enum TileKind { kTileStream16 = 0, kTileLds32 = 1, kTileLds128 = 2 };
+// with 32, 64 or 128.
+enum TileKind { kTileStream16 = 0, kTileLds32 = 1, kTileLds64 = 2, kTileLds128 = 3 };
 
 static int tile_bm(int kind) {
-    return kind == kTileStream16 ? 16 : (kind == kTileLds128 ? kQgBM : kQgBMSmall);
+    return kind == kTileStream16 ? 16
+           : kind == kTileLds32  ? kQgBMSmall
+           : kind == kTileLds64  ? kQgBMMid
+                                 : kQgBM;
 }
 
 // Tile choices, measured on MI355X.  A batch of at most 16 token rows streams
 // the weights (every task fits one row tile); the streaming tile needs
 // reductions that are whole multiples of 128 (`k128`).
 // MoE layer: 16-row streaming tile up to 16 rows (T = 8: 99 against 108 us
-// on the 32-row LDS tile), the 32-row LDS tile up to 80 rows per expert on
-// average (T = 64: 170 against 180 us streaming), 128 rows above.  Dense
-// projections: the 32-row tile up to 64 rows.
-static int moe_tile(int rows, double rows_per_expert, bool k128) {
+// on the 32-row LDS tile), then by the average rows per expert.  q8: the
+// 32-row tile up to 32 (T = 256: 212 us, 64-row 221, 128-row 229), the 64-row
+// tile, which copies the weights once where that takes two, up to 64 (T = 600:
+// 304, 278, 297), 128 rows above (T = 1400: 570, 471, 446).  q4: two 32-row
+// workgroups share a CU and win up to 140 (T = 600: 228, 250, 294; T = 1400:
+// 419, 430, 435; T = 2048: 572, 586, 557).  Dense projections: the 32-row
+// tile up to 64 rows.
+static int moe_tile(int fmt, int rows, double rows_per_expert, bool k128) {
     if (k128 && rows <= 16) return kTileStream16;
-    return rows_per_expert <= 80.0 ? kTileLds32 : kTileLds128;
+    if (fmt == kQ4) return rows_per_expert <= 140.0 ? kTileLds32 : kTileLds128;
+    return rows_per_expert <= 32.0 ? kTileLds32 : rows_per_expert <= 64.0 ? kTileLds64 : kTileLds128;
 }
 // Dense projections whose 128-row tiles would cover at most half the CUs
 // (o_proj and the dense down projection at 2048 rows: 128 tiles) take the
@@ -973,6 +994,7 @@ static int launch_qgemm_fmt(int fmt, bool dual, int kind, const QGemmLaunch &L, 
     switch (kind) {
     case kTileStream16: launch_stream_mb<1>(fmt, dual, L, grid, stream); break;
     case kTileLds32: launch_qgemm_bm<kQgBMSmall>(fmt, dual, L, grid, stream); break;
+    case kTileLds64: launch_qgemm_bm<kQgBMMid>(fmt, dual, L, grid, stream); break;
     case kTileLds128: launch_qgemm_bm<kQgBM>(fmt, dual, L, grid, stream); break;
     default: return kErrArgs;
     }
@@ -994,6 +1016,133 @@ int qgemm_single(int fmt, bool dual, const GemmTask &task, hipStream_t stream) {
     const int kind = dense_tile(task.rows, task.k % 128 == 0, task.n_out, dual);
     return launch_qgemm_fmt(fmt, dual, kind, L,
                             host_tiles(dual, task.rows, task.n_out, tile_bm(kind)), stream);
+}
+
+// ---------------------------------------------------------------------------
+// gemv() of many token rows
+// ---------------------------------------------------------------------------
+
+// Limb blocks and scales of one call's token rows: the library's own memory,
+// static, per GPU.  Launches of one GPU run in order on the library's one
+// stream, and a call's launches are queued under a lock, so no other call's
+// come between them; wider batches run in row chunks.  (No allocation: a call
+// may be captured.)
+constexpr long kTilesBytes = 64L << 20;
+constexpr int kTilesRows = 8192;
+constexpr int kTilesMaxWidth = 65536;  // int32 sums: 2^14 per column
+__device__ int8_t tiles_limbs[kTilesBytes];
+__device__ float tiles_scale[kTilesRows];
+static std::mutex tiles_mutex;
+
+// Four limbs of one row (x, or x * norm_w), a workgroup per row: step and split
+// as in gemv_batch.hip, over the whole row; the row's scale is the step times
+// 1 / rms, NaN where the row holds a NaN or an infinity.
+__global__ __launch_bounds__(256) void quantize4_kernel(const float *x, long x_stride, int width,
+                                                        const float *norm_w, float eps) {
+    __shared__ float red[2][4];
+    const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const float *xr = x + (long)row * x_stride;
+    float amax = 0.0f, ss = 0.0f;
+    auto load = [&](int i, float (&v)[4]) {
+        const f32x4 a = load_f4(xr + i);
+        v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w;
+    };
+    auto weigh = [&](int i, float (&v)[4]) {
+        if (!norm_w) return;
+        const f32x4 n = load_f4(norm_w + i);
+        v[0] *= n.x, v[1] *= n.y, v[2] *= n.z, v[3] *= n.w;
+    };
+    for (int i = tid * 4; i < width; i += 1024) {
+        float v[4];
+        load(i, v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ss = fmaf(v[e], v[e], ss);
+        weigh(i, v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) amax = __builtin_elementwise_maximum(amax, __builtin_fabsf(v[e]));
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        amax = __builtin_elementwise_maximum(amax, __shfl_xor(amax, o));
+        ss += __shfl_xor(ss, o);
+    }
+    if (lane == 0) red[0][wave] = amax, red[1][wave] = ss;
+    __syncthreads();
+    amax = __builtin_elementwise_maximum(__builtin_elementwise_maximum(red[0][0], red[0][1]),
+                                         __builtin_elementwise_maximum(red[0][2], red[0][3]));
+    const unsigned bits = __float_as_uint(amax) & 0x7FFFFFFFu;
+    const int ex = min(156 - (int)(bits >> 23), 126);  // amax 2^ex < 2^30
+    const float step_inv = __uint_as_float((unsigned)(127 + ex) << 23);
+    if (tid == 0) {
+        const float step = bits >= 0x7F800000u ? __builtin_nanf("")
+                                               : __uint_as_float((unsigned)(127 - ex) << 23);
+        const float tot = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+        tiles_scale[row] = norm_w ? step * (1.0f / sqrtf(tot / (float)width + eps)) : step;
+    }
+    int8_t *q = tiles_limbs + limb_at<4>(row, 0, width);
+    for (int i = tid * 4; i < width; i += 1024) {
+        float v[4];
+        load(i, v);
+        weigh(i, v);
+        unsigned l[4];
+        split_limbs4(v, step_inv, l[0], l[1], l[2], l[3]);
+#pragma unroll
+        for (int L = 0; L < 4; ++L)
+            *reinterpret_cast<unsigned *>(q + (i >> 7) * 4096 + L * 1024 + (i & 127)) = l[L];
+    }
+}
+
+bool gemv_tiles(const GemvParams &p, hipStream_t stream, std::string *name) {
+    const bool dual = p.epilogue == kEpiSiluDual;
+    auto al = [](const void *v) { return ((uintptr_t)v & 15u) == 0; };
+    if (!qgemm_shape_ok(p.fmt, p.I) || p.I > kTilesMaxWidth || p.limbs || p.router_parts || !al(p.w) ||
+        (dual && !al(p.w2)) || !al(p.x) || p.x_stride % 4 || (p.norm_w && !al(p.norm_w)))
+        return false;
+    if (name) {
+        char buf[64];
+        snprintf(buf, sizeof(buf), "mlh::qgemm_kernel<%d, %s, %d, 4>", p.fmt, dual ? "true" : "false",
+                 kQgBMMid);
+        *name = buf;
+        return true;
+    }
+    static int8_t *limbs[64] = {};  // device addresses, looked up once per GPU
+    static float *scale[64] = {};
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return false;
+    const std::lock_guard<std::mutex> lock(tiles_mutex);
+    if (!limbs[device] &&
+        (hipGetSymbolAddress((void **)&scale[device], HIP_SYMBOL(tiles_scale)) != hipSuccess ||
+         hipGetSymbolAddress((void **)&limbs[device], HIP_SYMBOL(tiles_limbs)) != hipSuccess)) {
+        (void)hipGetLastError();  // not sticky: the caller falls back
+        return false;
+    }
+    long chunk = std::min<long>(kTilesRows, kTilesBytes / limb_row_block<4>(p.I) * 8);
+    for (long r0 = 0; r0 < p.rows; r0 += chunk) {
+        const int n = (int)std::min<long>(chunk, p.rows - r0);
+        hipLaunchKernelGGL(quantize4_kernel, dim3(n), dim3(256), 0, stream, p.x + r0 * p.x_stride,
+                           p.x_stride, p.I, p.norm_w, p.eps);
+        QGemmLaunch L;
+        GemmTask &t = L.single;
+        t.w = p.w;
+        t.s = p.s;
+        t.w2 = p.w2;
+        t.s2 = p.s2;
+        t.rows = n;
+        t.n_out = p.O;
+        t.k = p.I;
+        t.a = limbs[device];
+        t.a_width = p.I;
+        t.a_scale = scale[device];
+        t.y = p.y + r0 * p.y_stride;
+        t.y_stride = p.y_stride;
+        if (p.epilogue == kEpiResidual) {
+            t.resid = p.resid + r0 * p.resid_stride;
+            t.resid_stride = p.resid_stride;
+        }
+        const int tiles = host_tiles(dual, n, p.O, kQgBMMid);
+        launch_qgemm_bm<kQgBMMid, 4>(p.fmt, dual, L, (tiles + 7) / 8 * 8, stream);
+    }
+    return true;
 }
 
 // ---------------------------------------------------------------------------
@@ -1185,7 +1334,8 @@ int moe_gemm(const MoeGemmParams &p, hipStream_t stream) {
     // one tile kind for the whole layer, from the average rows per expert
     const bool k128 = p.hidden % 128 == 0 && p.inter % 128 == 0 &&
                       (!p.has_shared || p.shared_width % 128 == 0);
-    const int kind = moe_tile(p.rows, (double)entries / p.experts, k128);
+    const int fmt = p.expert_fmt == kQ8 || (p.has_shared && p.shared_fmt == kQ8) ? kQ8 : kQ4;
+    const int kind = moe_tile(fmt, p.rows, (double)entries / p.experts, k128);
     const int bm = tile_bm(kind);
     MoeScheduleParams sp;
     sp.p = p;

@@ -914,20 +914,16 @@ bool to_host(MoonlightSession *s, void *dst, const void *src, size_t bytes) {
 // routing in its first launch, while the grouped GEMV runs a routing launch,
 // two stage launches and a combine (measured on MI355X, whole layer: equal at
 // T = 2, 53.5 us; 58 against 74 us at T = 3, 64 against 92 us at T = 4).
-// The dense projections take it where the batch kernel (gemv_batch.hip, one
-// launch, x split in every workgroup) would need more than kBatchMaxGroups
-// workgroups of 64 weight rows, 16 token rows and 2048 columns: two rounds of
-// the CUs.
+// The dense projections take it where the batch kernel does not fit
+// (gemv_batch_fits).
 constexpr int kGemmMinRows = 16;
 constexpr int kMoeGemmMinRows = 3;
-constexpr long kBatchMaxGroups = 512;
 
 // out_w: weight rows of the launch (a SwiGLU pair: gate and up).
 bool use_gemm(const MoonlightSession *s, int fmt, int rows, int in_w, int out_w) {
     if (rows < kGemmMinRows || !s->aq || in_w > s->aq_width || !qgemm_shape_ok(fmt, in_w))
         return false;
-    const long groups = ((long)out_w + 63) / 64 * ((rows + 15) / 16) * ((in_w + 2047) / 2048);
-    return groups > kBatchMaxGroups;
+    return !gemv_batch_fits(out_w, rows, in_w);
 }
 
 int gemm_rows(MoonlightSession *s, const Matrix &m, const Matrix *up, const float *x, int rows,

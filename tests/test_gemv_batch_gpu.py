@@ -43,6 +43,22 @@ SHAPES = [
 def test_batch_matches_oracle(device, fmt, out_width, in_width, rows):
     print(f"[gpu] batch fmt={fmt} O={out_width} I={in_width} rows={rows}", flush=True)
     assert "gemv_batch_kernel" in native.gemv_kernel_name(fmt, out_width, in_width, rows)
+    check(fmt, out_width, in_width, rows)
+
+
+# the four-limb GEMM tiles (qgemm.hip) that larger batches take: row tiles of 64
+# and column tiles of 256 with remainders, widths that end inside a 128-wide
+# slice, and a width whose rows take more than one scratch chunk
+@pytest.mark.parametrize("fmt", [1, 2])
+@pytest.mark.parametrize("out_width,in_width,rows", [
+    (11264, 2048, 97), (4100, 64, 300), (3001, 2112, 321), (900, 192, 1100), (5000, 16448, 260)])
+def test_tiles_match_oracle(device, fmt, out_width, in_width, rows):
+    print(f"[gpu] tiles fmt={fmt} O={out_width} I={in_width} rows={rows}", flush=True)
+    assert "qgemm_kernel" in native.gemv_kernel_name(fmt, out_width, in_width, rows)
+    check(fmt, out_width, in_width, rows)
+
+
+def check(fmt, out_width, in_width, rows):
     q, s = make_weights(fmt, out_width, in_width, seed=out_width + in_width)
     x = O.fill_normal(rows * in_width, 31 + rows).reshape(rows, in_width)
     nw = O.fill_normal(in_width, 4, mean=1.0, std=0.1)
@@ -61,7 +77,8 @@ def test_batch_matches_oracle(device, fmt, out_width, in_width, rows):
 
 @pytest.mark.parametrize("fmt", [1, 2])
 @pytest.mark.parametrize("width,in_width,rows", [
-    (40, 96, 3), (100, 2048, 7), (1408, 4096, 16), (9000, 64, 17), (33, 999, 6)])
+    (40, 96, 3), (100, 2048, 7), (1408, 4096, 16), (9000, 64, 17), (33, 999, 6),
+    (2816, 192, 200)])  # GEMM tiles
 def test_batch_swiglu(device, fmt, width, in_width, rows):
     print(f"[gpu] batch swiglu fmt={fmt} W={width} I={in_width} rows={rows}", flush=True)
     (qg, sg), (qu, su) = (make_weights(fmt, width, in_width, seed=k) for k in (21, 22))
@@ -92,11 +109,11 @@ def test_batch_unaligned_operands(device, fmt, rows, w_off, x_off):
     assert rel_l2(dy.download(np.float32).reshape(rows, out_width), expect) < TOL
 
 
-@pytest.mark.parametrize("fmt,in_width", [(1, 2048), (2, 4103)])
-def test_batch_nonfinite_inputs(device, fmt, in_width):
+@pytest.mark.parametrize("fmt,out_width,in_width,rows", [
+    (1, 48, 2048, 6), (2, 48, 4103, 6), (1, 9000, 1024, 110)])  # the last: GEMM tiles
+def test_batch_nonfinite_inputs(device, fmt, out_width, in_width, rows):
     """A NaN or infinity anywhere in a token row, the cut end included, leaves
     no finite output in it and the other rows untouched."""
-    out_width, rows = 48, 6
     q, s = make_weights(fmt, out_width, in_width, seed=8)
     x = O.fill_normal(rows * in_width, 6).reshape(rows, in_width)
     x[0, 3], x[2, in_width - 1], x[3, 1000] = np.inf, np.nan, -np.inf
@@ -104,6 +121,6 @@ def test_batch_nonfinite_inputs(device, fmt, in_width):
     dy = DeviceBuffer(rows * out_width * 4)
     native.gemv(fmt, dw, ds, dx, dy, out_width, in_width, rows)
     got = dy.download(np.float32).reshape(rows, out_width)
-    fine = [1, 4, 5]
+    fine = [r for r in range(rows) if r not in (0, 2, 3)]
     assert not np.isfinite(got[[0, 2, 3]]).any()
     assert rel_l2(got[fine], O.matmul(fmt, q, s, x[fine], out_width, in_width)) < TOL
