@@ -261,6 +261,8 @@ int gemv_rows_per_block(const GemvPlan &plan, bool dual) {
 
 bool gemv_mfma(const GemvParams &p, hipStream_t stream, std::string *name = nullptr);  // gemv_mfma.hip
 bool gemv_batch(const GemvParams &p, hipStream_t stream, std::string *name = nullptr);  // gemv_batch.hip
+bool gemv_f32_batch(const GemvParams &p, hipStream_t stream,
+                    std::string *name = nullptr);  // gemv_f32_batch.hip
 
 static bool aligned16(const void *ptr) { return ((uintptr_t)ptr & 15u) == 0; }
 
@@ -290,7 +292,7 @@ std::string gemv_kernel_name(int fmt, int O, int I, int rows, bool dual) {
     q.epilogue = dual ? kEpiSiluDual : q.epilogue;
     std::string mfma;
     q.x_stride = I;
-    if (gemv_mfma(q, nullptr, &mfma) ||
+    if (gemv_mfma(q, nullptr, &mfma) || gemv_f32_batch(q, nullptr, &mfma) ||
         (q.rows > 4 && !gemv_batch_fits(q) && gemv_tiles(q, nullptr, &mfma)) || (!vector_first(q, vector_takes(q)) && gemv_batch(q, nullptr, &mfma)))
         return mfma;
     const GemvPlan pl = plan_gemv(fmt, O, I, rows < kMaxGemvRows ? rows : kMaxGemvRows, dual);
@@ -314,7 +316,7 @@ int gemv(const GemvParams &p_in, hipStream_t stream) {
          !gemv_router_ok(p_in)))
         return kErrArgs;
     // q8 / q4 with up to 4 token rows: the matrix-core kernel when it takes the shape
-    if (gemv_mfma(p_in, stream))
+    if (gemv_mfma(p_in, stream) || gemv_f32_batch(p_in, stream))
         return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
     if (p_in.router_parts) return kErrArgs;
     if (p_in.rows > 4 && !gemv_batch_fits(p_in) && gemv_tiles(p_in, stream))

@@ -1,6 +1,7 @@
-"""GPU parity of the batch dequant matmul (gemv_batch.hip: q8 / q4, any width,
-from 2 token rows where the one-pass kernels of gemv_mfma.hip do not take the
-shape) against the CPU oracle, at the edges of its tiles.
+"""GPU parity of the matmuls of several token rows (gemv_batch.hip: q8 / q4, any
+width, from 2 token rows where the one-pass kernels of gemv_mfma.hip do not take
+the shape; gemv_f32_batch.hip; the GEMM tiles of larger batches) against the CPU
+oracle, at the edges of their tiles.
 
 Tolerance: x is split exactly to 30 bits and every product is exact, so the
 difference is the oracle's own serial fp32 sum: at most I * 2^-24 relative, in
@@ -71,6 +72,30 @@ def check(fmt, out_width, in_width, rows):
         native.gemv(fmt, dw, ds, dx, dy, out_width, in_width, rows, norm_w=norm, eps=1e-5,
                     resid=resid)
         expect = O.matmul(fmt, q, s, xn if norm else x, out_width, in_width)
+        got = dy.download(np.float32).reshape(rows, out_width)
+        assert rel_l2(got, res + expect if resid else expect) < TOL
+
+
+# f32 matrices of many rows: token tiles of 4, 8 and 16 with remainders, weight
+# tiles of 64 and 32 with remainders, rows of fewer and more chunks than a
+# wave's two loads, widths whose token rows fill the LDS
+@pytest.mark.parametrize("out_width,in_width,rows,norm", [
+    (4096, 2048, 3, True), (4099, 4, 4, True), (8200, 252, 5, False), (8193, 260, 8, False),
+    (9001, 516, 9, True), (8192, 2048, 17, False), (4100, 4096, 12, True), (4097, 9216, 4, True)])
+def test_f32_batch_matches_oracle(device, out_width, in_width, rows, norm):
+    print(f"[gpu] f32 batch O={out_width} I={in_width} rows={rows}", flush=True)
+    w, _ = make_weights(0, out_width, in_width, seed=out_width + in_width)
+    x = O.fill_normal(rows * in_width, 31 + rows).reshape(rows, in_width)
+    nw = O.fill_normal(in_width, 4, mean=1.0, std=0.1)
+    res = O.fill_normal(rows * out_width, 9).reshape(rows, out_width)
+    xn = np.empty_like(x)
+    O.lib().orc_rmsnorm(O.fptr(x), O.fptr(nw), O.fptr(xn), rows, in_width, 1e-5)
+    dw, dx, dn, dr = (DeviceBuffer.from_array(a) for a in (w, x, nw, res))
+    dy = DeviceBuffer(rows * out_width * 4)
+    expect = O.matmul(0, w, None, xn if norm else x, out_width, in_width)
+    for resid in (None, dr):
+        native.gemv(0, dw, None, dx, dy, out_width, in_width, rows, norm_w=dn if norm else None,
+                    eps=1e-5, resid=resid)
         got = dy.download(np.float32).reshape(rows, out_width)
         assert rel_l2(got, res + expect if resid else expect) < TOL
 
