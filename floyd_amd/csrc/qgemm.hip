@@ -959,6 +959,11 @@ static int tile_bm(int kind) {
                                  : kQgBM;
 }
 
+static int host_tiles(bool dual, int rows, int n_out, int bm) {
+    const int outw = dual ? kQgBW / 2 : kQgBW;
+    return ((rows + bm - 1) / bm) * ((n_out + outw - 1) / outw);
+}
+
 // Tile choices, measured on MI355X.  A batch of at most 16 token rows streams
 // the weights (every task fits one row tile); the streaming tile needs
 // reductions that are whole multiples of 128 (`k128`).
@@ -968,22 +973,21 @@ static int tile_bm(int kind) {
 // tile, which copies the weights once where that takes two, up to 64 (T = 600:
 // 304, 278, 297), 128 rows above (T = 1400: 570, 471, 446).  q4: two 32-row
 // workgroups share a CU and win up to 140 (T = 600: 228, 250, 294; T = 1400:
-// 419, 430, 435; T = 2048: 572, 586, 557).  Dense projections: the 32-row
-// tile up to 64 rows.
+// 419, 430, 435; T = 2048: 572, 586, 557).
 static int moe_tile(int fmt, int rows, double rows_per_expert, bool k128) {
     if (k128 && rows <= 16) return kTileStream16;
     if (fmt == kQ4) return rows_per_expert <= 140.0 ? kTileLds32 : kTileLds128;
     return rows_per_expert <= 32.0 ? kTileLds32 : rows_per_expert <= 64.0 ? kTileLds64 : kTileLds128;
 }
-// Dense projections whose 128-row tiles would cover at most half the CUs
-// (o_proj and the dense down projection at 2048 rows: 128 tiles) take the
-// 32-row tile too: 52.8 against 58.4 us for o_proj at 2048 rows; at 240
-// tiles (`[q; kv_a]`) the 32-row tile measured 75.1 against 51.1 us.
+// Dense projections: the smallest tile that covers the matrix in one round of
+// the CUs, else 128 rows.  Tiles of 32 / 64 / 128 rows: 2048 x 2048 at 600 rows
+// 19.8 / 23.9 / 36.4 us, at 1200 rows 36.8 / 27.5 / 39.1, at 2048 rows 42.4 /
+// 31.1 / 45.0; 3648 x 2048 at 600 rows 34.9 / 25.0 / 37.9, at 1200 rows 52.2 /
+// 48.0 / 41.0, at 2048 rows 76.4 / 57.8 / 48.6.
 static int dense_tile(int rows, bool k128, int n_out, bool dual) {
     if (k128 && rows <= 16) return kTileStream16;
-    const int outw = dual ? kQgBW / 2 : kQgBW;
-    const long t128 = (long)((rows + kQgBM - 1) / kQgBM) * ((n_out + outw - 1) / outw);
-    return rows <= 2 * kQgBMSmall || t128 <= 128 ? kTileLds32 : kTileLds128;
+    if (host_tiles(dual, rows, n_out, kQgBMSmall) <= 256) return kTileLds32;
+    return host_tiles(dual, rows, n_out, kQgBMMid) <= 256 ? kTileLds64 : kTileLds128;
 }
 
 static int launch_qgemm_fmt(int fmt, bool dual, int kind, const QGemmLaunch &L, int tiles_bound,
@@ -999,11 +1003,6 @@ static int launch_qgemm_fmt(int fmt, bool dual, int kind, const QGemmLaunch &L, 
     default: return kErrArgs;
     }
     return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
-}
-
-static int host_tiles(bool dual, int rows, int n_out, int bm) {
-    const int outw = dual ? kQgBW / 2 : kQgBW;
-    return ((rows + bm - 1) / bm) * ((n_out + outw - 1) / outw);
 }
 
 int qgemm_single(int fmt, bool dual, const GemmTask &task, hipStream_t stream) {
