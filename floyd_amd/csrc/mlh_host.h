@@ -68,8 +68,17 @@ inline bool gemv_batch_fits(long weight_rows, int rows, int in_width) {
     const long chunks = (in_width + 2047) / 2048;
     return (weight_rows + 63) / 64 * ((rows + 15) / 16) * chunks <= 300 + 600 * chunks;
 }
+// The same for a gemv() call: its tiles split a long reduction over the CUs
+// (SwiGLU pairs don't) and then take 37 us for 4096 columns, 41 for 6144, 44 for
+// 8192 and 48 for 11264.  Batch against tiles: 2048 x 4096 at 200 rows 37.1 / 36.5
+// us, at 350 54.9 / 38.4; 2048 x 6144 at 150 49.6 / 40.1; 2048 x 8192 at 100 32.9 /
+// 42.1, at 200 63.8 / 44.1; 2048 x 11264 at 96 43.4 / 47.8, at 192 84.5 / 49.1;
+// 576 x 11264 at 200 28.6 / 50.8, at 700 86.5 / 59.0.
 inline bool gemv_batch_fits(const GemvParams &p) {
-    return gemv_batch_fits((long)p.O * (p.epilogue == kEpiSiluDual ? 2 : 1), p.rows, p.I);
+    const long chunks = (p.I + 2047) / 2048;
+    if (p.epilogue == kEpiSiluDual || chunks == 1)
+        return gemv_batch_fits((long)p.O * (p.epilogue == kEpiSiluDual ? 2 : 1), p.rows, p.I);
+    return ((long)p.O + 63) / 64 * ((p.rows + 15) / 16) * chunks <= 600 + 110 * chunks;
 }
 // Whether gemv() can write router logit partials for p (router fields
 // aside), and how many partials per expert it then writes.

@@ -81,6 +81,7 @@ struct QGemmLaunch {
     const int *n_routed = nullptr;    // device: routed task count (shared tasks follow)
     int n_shared = 1;                 // shared-expert tasks after the routed ones
     int range = 0;                    // 0 all tasks, 1 routed only, 2 shared only
+    int splits = 1;                   // shares of `single`'s reduction
     GemmTask single;
 };
 

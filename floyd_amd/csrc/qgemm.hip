@@ -250,9 +250,14 @@ __host__ __device__ __forceinline__ int tiles_of(int rows, int n_out) {
 // Tiles run in XCD-contiguous order (workgroup i goes to XCD i % 8): each XCD
 // takes a contiguous range of tiles, and within a task groups of kQgGroup row
 // tiles share one column tile, so neighbouring workgroups of an XCD reuse
-// weight tiles from its L2.
-template <bool DUAL, int BM>
-__device__ __forceinline__ bool map_tile(const QGemmLaunch &L, GemmTask &tk, int &m0, int &n0) {
+// weight tiles from its L2.  SPLIT: every tile once per share of the reduction,
+// all tiles of a share one after the other; tile and share numbers in at.
+struct SplitAt {
+    int tile = 0, share = 0;
+};
+template <bool DUAL, int BM, bool SPLIT = false>
+__device__ __forceinline__ bool map_tile(const QGemmLaunch &L, GemmTask &tk, int &m0, int &n0,
+                                         SplitAt *at = nullptr) {
     int local;
     {
         int begin = 0, end;
@@ -263,7 +268,7 @@ __device__ __forceinline__ bool map_tile(const QGemmLaunch &L, GemmTask &tk, int
             end = L.range == 1 ? L.tile_start[nr] : L.tile_start[nr + L.n_shared];
             if (L.range == 2) begin = L.tile_start[nr];
         } else {
-            end = tiles_of<DUAL, BM>(L.single.rows, L.single.n_out);
+            end = tiles_of<DUAL, BM>(L.single.rows, L.single.n_out) * (SPLIT ? L.splits : 1);
         }
         const int total = end - begin;
         const int per = (total + 7) >> 3;
@@ -278,6 +283,11 @@ __device__ __forceinline__ bool map_tile(const QGemmLaunch &L, GemmTask &tk, int
         } else {
             tk = L.single;
             local = tile;
+        }
+        if constexpr (SPLIT) {
+            const int tiles = end / L.splits;
+            at->share = local / tiles;
+            at->tile = local -= at->share * tiles;
         }
     }
     constexpr int outw = DUAL ? kQgBW / 2 : kQgBW;
@@ -384,10 +394,23 @@ __device__ __forceinline__ float silu_times(float g, float u) {
     return fmaf(fmaf(-d, q, n), r, q);
 }
 
+// Shares of a split reduction (the library's own memory, static, per GPU:
+// launches of one GPU run in order on the library's one stream).  A share is
+// the exact integer sum of its tile's limb products, as a double (at most 2^53
+// at the four-limb tiles' widths), so the total does not depend on the split.
+constexpr int kSplitMaxShares = 256;              // workgroups of a split launch
+constexpr int kSplitTile = kQgBMMid * kQgBW;      // outputs of its tiles
+constexpr int kSplitCountStride = 32;             // ints between counters (128 bytes)
+__device__ double split_part[(long)kSplitMaxShares * kSplitTile];
+__device__ int split_count[kSplitMaxShares * kSplitCountStride];  // zero between launches
+
 // Workgroup over a BM x 256 tile (QgShape).  The 32-row tile serves
 // batches whose experts hold few rows each: the MFMA work per weight byte is
 // a quarter, so the tile is bound by the weight stream instead of by padding.
-template <int FMT, bool DUAL, int BM, int LIMBS>
+// SPLIT: over one share of the tile's reduction (whole slices, L.splits shares
+// of as equal length as they go); the workgroup that arrives last adds the
+// other shares to its own and writes the outputs.
+template <int FMT, bool DUAL, int BM, int LIMBS, bool SPLIT>
 __global__ __launch_bounds__((QgShape<FMT, BM, LIMBS>::kThreads),
                              (BM != 32 || FMT == kQ8) ? 1 : 2) void qgemm_kernel(QGemmLaunch L) {
     extern __shared__ __attribute__((aligned(16))) int8_t qg_lds[];
@@ -400,7 +423,19 @@ __global__ __launch_bounds__((QgShape<FMT, BM, LIMBS>::kThreads),
     float *lds_scale = reinterpret_cast<float *>(qg_lds);  // after the products
     GemmTask tk;
     int m0, n0;
-    if (!map_tile<DUAL, BM>(L, tk, m0, n0)) return;
+    SplitAt at;
+    if (!map_tile<DUAL, BM, SPLIT>(L, tk, m0, n0, &at)) return;
+    long w_skip = 0;  // bytes of a weight row before the share
+    if constexpr (SPLIT) {
+        static_assert(!DUAL && BM * kQgBW == kSplitTile, "one sum per output, the shares' layout");
+        const int slices = (tk.k + kQgSlice - 1) / kQgSlice;
+        const int first = slices * at.share / L.splits, last = slices * (at.share + 1) / L.splits;
+        w_skip = (long)first * kRBB;
+        tk.w_ld = tk.k;
+        tk.w += w_skip;
+        tk.a += (long)first * (LIMBS * 1024);
+        tk.k = min(tk.k, last * kQgSlice) - first * kQgSlice;
+    }
 
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
@@ -432,7 +467,7 @@ __global__ __launch_bounds__((QgShape<FMT, BM, LIMBS>::kThreads),
     const int8_t *const a_base = tk.a + limb_at<LIMBS>(a_first, 0, tk.a_width);
     const uint8_t *const w_base = tk.w + n0 * w_row_bytes;
     const uint8_t *const w2_base = DUAL ? tk.w2 + n0 * w_row_bytes : nullptr;
-    const long w_bytes = (tk.n_out - n0) * w_row_bytes;
+    const long w_bytes = (tk.n_out - n0) * w_row_bytes - w_skip;
     // weight row from n0 held by LDS B row j: SwiGLU tiles give each wave its kNF / 2
     // gate blocks and then the matching up blocks (kNF = 4: blocks f = 0, 1
     // gate, 2, 3 up of a 128-row wave half; kNF = 2: block 0 gate, 1 up of a
@@ -605,6 +640,49 @@ __global__ __launch_bounds__((QgShape<FMT, BM, LIMBS>::kThreads),
         for (int ks = 1; ks < nk; ++ks) next_slice(ks);
     }
 
+    // ---- shares: stored, and added by the tile's last workgroup
+    double total[SPLIT ? kNF : 1][16];
+    if constexpr (SPLIT) {
+        constexpr int kShift = FMT == kQ4 ? 4 : 0;
+#pragma unroll
+        for (int f = 0; f < kNF; ++f)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                double v = acc[0][f][r] >> kShift;
+#pragma unroll
+                for (int a = 1; a < LIMBS; ++a) v = fma(v, 256.0, (double)(acc[a][f][r] >> kShift));
+                total[f][r] = v;
+            }
+        auto part_of = [&](int share) {
+            return split_part + (long)(at.tile * L.splits + share) * kSplitTile + tid;
+        };
+        if (live) {
+            double *part = part_of(at.share);
+#pragma unroll
+            for (int f = 0; f < kNF; ++f)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    __hip_atomic_store(part + (f * 16 + r) * Sh::kThreads, total[f][r], __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+        }
+        int *count = split_count + at.tile * kSplitCountStride;
+        if (!agent_handoff_arrive(count, L.splits)) return;
+        if (tid == 0) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (live) {
+            for (int share = 0; share < L.splits; ++share) {
+                if (share == at.share) continue;
+                const double *part = part_of(share);
+                double v[kNF * 16];
+#pragma unroll
+                for (int i = 0; i < kNF * 16; ++i)
+                    v[i] = __hip_atomic_load(part + i * Sh::kThreads, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                for (int i = 0; i < kNF * 16; ++i) total[i / 16][i % 16] += v[i];
+            }
+        }
+    }
+
     // ---- epilogue, without a branch: stores and residual loads go through
     // buffers of the tile's own rows, so rows past the task's end are out of
     // range (dropped, read as zero), as are the columns past n_out, whose
@@ -634,6 +712,7 @@ __global__ __launch_bounds__((QgShape<FMT, BM, LIMBS>::kThreads),
     // the limbs' sum of one result register, 256 apart (the int32 sums are
     // exact; q4 ones are 16 times the products')
     auto limb_sum = [&](int f, int r) -> float {
+        if constexpr (SPLIT) return (float)total[f][r];
         constexpr int kShift = FMT == kQ4 ? 4 : 0;
         float v = (float)(acc[LIMBS - 1][f][r] >> kShift), unit = 1.0f;
 #pragma unroll
@@ -898,16 +977,16 @@ __global__ __launch_bounds__(256, 2) void qgemm_stream_kernel(QGemmLaunch L) {
         }
 }
 
-template <int FMT, bool DUAL, int BM, int LIMBS = kLimbs>
+template <int FMT, bool DUAL, int BM, int LIMBS = kLimbs, bool SPLIT = false>
 static void launch_qgemm(const QGemmLaunch &L, int grid, hipStream_t stream) {
     using Sh = QgShape<FMT, BM, LIMBS>;
     static const bool attr = [] {
-        return hipFuncSetAttribute(reinterpret_cast<const void *>(&qgemm_kernel<FMT, DUAL, BM, LIMBS>),
+        return hipFuncSetAttribute(reinterpret_cast<const void *>(&qgemm_kernel<FMT, DUAL, BM, LIMBS, SPLIT>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize,
                                    Sh::kLds) == hipSuccess;
     }();
     (void)attr;
-    hipLaunchKernelGGL((qgemm_kernel<FMT, DUAL, BM, LIMBS>), dim3((unsigned)grid), dim3(Sh::kThreads),
+    hipLaunchKernelGGL((qgemm_kernel<FMT, DUAL, BM, LIMBS, SPLIT>), dim3((unsigned)grid), dim3(Sh::kThreads),
                        Sh::kLds, stream, L);
 }
 
@@ -1091,6 +1170,24 @@ __global__ __launch_bounds__(256) void quantize4_kernel(const float *x, long x_s
     }
 }
 
+// Token rows of one launch.
+static long tiles_chunk(const GemvParams &p) {
+    return std::min<long>(std::min<long>(kTilesRows, kTilesBytes / limb_row_block<4>(p.I) * 8), p.rows);
+}
+
+// Shares of the reduction: as many as keep the launch in one round of the CUs
+// (a 2048-row matrix has 8 tiles per 64 token rows), none shorter than
+// kSplitMinSlices slices (2048 columns), where storing and adding the shares (128
+// KB each) costs as much as it saves.  2048 x 11264 at 777 rows (104 tiles,
+// 2 shares) 139 -> 96 us, at 330 rows (48 tiles, 5 shares) 120 -> 60.
+constexpr int kSplitMinSlices = 16;
+static int tile_splits(const GemvParams &p, long rows) {
+    if (p.epilogue == kEpiSiluDual) return 1;
+    const long tiles = host_tiles(false, (int)rows, p.O, kQgBMMid);
+    const long fit = kSplitMaxShares / tiles, slices = (p.I + kQgSlice - 1) / kQgSlice;
+    return (int)std::max<long>(1, std::min<long>(fit, slices / kSplitMinSlices));
+}
+
 bool gemv_tiles(const GemvParams &p, hipStream_t stream, std::string *name) {
     const bool dual = p.epilogue == kEpiSiluDual;
     auto al = [](const void *v) { return ((uintptr_t)v & 15u) == 0; };
@@ -1099,8 +1196,8 @@ bool gemv_tiles(const GemvParams &p, hipStream_t stream, std::string *name) {
         return false;
     if (name) {
         char buf[64];
-        snprintf(buf, sizeof(buf), "mlh::qgemm_kernel<%d, %s, %d, 4>", p.fmt, dual ? "true" : "false",
-                 kQgBMMid);
+        snprintf(buf, sizeof(buf), "mlh::qgemm_kernel<%d, %s, %d, 4, %s>", p.fmt,
+                 dual ? "true" : "false", kQgBMMid, tile_splits(p, tiles_chunk(p)) > 1 ? "true" : "false");
         *name = buf;
         return true;
     }
@@ -1115,7 +1212,7 @@ bool gemv_tiles(const GemvParams &p, hipStream_t stream, std::string *name) {
         (void)hipGetLastError();  // not sticky: the caller falls back
         return false;
     }
-    long chunk = std::min<long>(kTilesRows, kTilesBytes / limb_row_block<4>(p.I) * 8);
+    const long chunk = tiles_chunk(p);
     for (long r0 = 0; r0 < p.rows; r0 += chunk) {
         const int n = (int)std::min<long>(chunk, p.rows - r0);
         hipLaunchKernelGGL(quantize4_kernel, dim3(n), dim3(256), 0, stream, p.x + r0 * p.x_stride,
@@ -1138,8 +1235,11 @@ bool gemv_tiles(const GemvParams &p, hipStream_t stream, std::string *name) {
             t.resid = p.resid + r0 * p.resid_stride;
             t.resid_stride = p.resid_stride;
         }
-        const int tiles = host_tiles(dual, n, p.O, kQgBMMid);
-        launch_qgemm_bm<kQgBMMid, 4>(p.fmt, dual, L, (tiles + 7) / 8 * 8, stream);
+        L.splits = tile_splits(p, n);
+        const int grid = (host_tiles(dual, n, p.O, kQgBMMid) * L.splits + 7) / 8 * 8;
+        if (L.splits == 1) launch_qgemm_bm<kQgBMMid, 4>(p.fmt, dual, L, grid, stream);
+        else if (p.fmt == kQ8) launch_qgemm<kQ8, false, kQgBMMid, 4, true>(L, grid, stream);
+        else launch_qgemm<kQ4, false, kQgBMMid, 4, true>(L, grid, stream);
     }
     return true;
 }
