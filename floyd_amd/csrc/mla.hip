@@ -1219,6 +1219,12 @@ __global__ __launch_bounds__(256, 2) void mla_expand_kernel(MlaParams p) {
 // on 4 waves exceed the register file.
 constexpr int kPfRowsPerGroup = 2;
 constexpr int kPfWaves = 4;
+// Up to as many rows as CUs, where a workgroup per row still leaves none waiting:
+// 1 row on 8 waves, which halves a wave's part of every tile (the serial chain
+// over the tiles is the bound) and the code that a short launch fetches.  2 rows
+// on 4 waves against it: 8 rows at position 0 14.3 / 7.9 us, 63 rows 24.1 / 14.2; 8
+// rows at 1024 226 / 135, 32 rows at 4096 879 / 523.
+constexpr int kPfFewRows = 256;
 constexpr int kPfKeys = 16;
 constexpr int kPfRowStride = kMlaMaxLatent + 4;  // latent rows in LDS (rope in registers)
 // The running max of a (row, head) moves only when a tile's max exceeds it
@@ -1955,6 +1961,17 @@ static bool mla_prefill_expanded(const MlaParams &p, hipStream_t stream) {
 // short prompt (more rows come here only with keys past the expanded copy).
 constexpr int kValueFewRows = 64;
 
+template <int RB, int NW>
+static void launch_prefill_attend(const MlaParams &p, hipStream_t stream) {
+    constexpr size_t lds = pf_lds_bytes<RB, NW>();
+    static const bool attr =
+        hipFuncSetAttribute(reinterpret_cast<const void *>(&mla_prefill_attend_kernel<RB, NW>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+    (void)attr;
+    hipLaunchKernelGGL((mla_prefill_attend_kernel<RB, NW>), dim3((p.rows + RB - 1) / RB),
+                       dim3(64 * NW), lds, stream, p);
+}
+
 int mla_attention_core(const MlaParams &p, hipStream_t stream) {
     if (p.heads <= 0 || p.heads > kMlaMaxHeads || p.latent <= 0 || p.latent % 64 ||
         p.latent > kMlaMaxLatent || p.rope <= 0 || p.rope > 64 || (p.rope & 1) ||
@@ -1968,11 +1985,6 @@ int mla_attention_core(const MlaParams &p, hipStream_t stream) {
     if (p.rows > 1 && !p.grid_splits && p.nope % 16 == 0 && p.vdim % 16 == 0) {
         // prefill: cache append + query rope, the absorb as a per-head GEMM,
         // flash attention writing lc directly, the value as a per-head GEMM
-        constexpr int RB = kPfRowsPerGroup, NW = kPfWaves;
-        static const bool attr = hipFuncSetAttribute(
-            reinterpret_cast<const void *>(&mla_prefill_attend_kernel<RB, NW>),
-            hipFuncAttributeMaxDynamicSharedMemorySize, (int)pf_lds_bytes<RB, NW>()) == hipSuccess;
-        (void)attr;
         const unsigned mt = (unsigned)((p.rows + 63) / 64);
         // the cache rows and every head's query rope, one workgroup a row
         // (measured on MI355X, 2048-token prefill: 12.5 us per layer against
@@ -1988,8 +2000,8 @@ int mla_attention_core(const MlaParams &p, hipStream_t stream) {
         const bool fa = (q8 && launch_head_gemm_f16<kHgAbsorb, kQ8>(p, ga, stream)) ||
                         (q4 && launch_head_gemm_f16<kHgAbsorb, kQ4>(p, ga, stream));
         if (!fa) hipLaunchKernelGGL(mla_head_gemm_kernel<true>, ga, dim3(256), 0, stream, p);
-        hipLaunchKernelGGL((mla_prefill_attend_kernel<RB, NW>), dim3((p.rows + RB - 1) / RB),
-                           dim3(64 * NW), (pf_lds_bytes<RB, NW>()), stream, p);
+        if (p.rows <= kPfFewRows) launch_prefill_attend<1, 8>(p, stream);
+        else launch_prefill_attend<kPfRowsPerGroup, kPfWaves>(p, stream);
         if ((q8 || q4) && p.latent == 512 && p.rows <= kValueFewRows) {
             const dim3 gf((unsigned)((p.rows + 15) / 16), (unsigned)((p.vdim + 15) / 16),
                           (unsigned)p.heads);
