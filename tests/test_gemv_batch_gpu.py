@@ -49,12 +49,12 @@ def test_batch_matches_oracle(device, fmt, out_width, in_width, rows):
 
 # the four-limb GEMM tiles (qgemm.hip) that larger batches take: row tiles of 64
 # and column tiles of 256 with remainders, widths that end inside a 128-wide
-# slice, and a width whose rows take more than one scratch chunk; reductions in 2,
-# 5 and 10 shares, the last of them ending inside a slice
+# slice, and a width whose rows take more than one scratch chunk; reductions in 2
+# shares, the last of them ending inside a slice, and in 5
 @pytest.mark.parametrize("fmt", [1, 2])
 @pytest.mark.parametrize("out_width,in_width,rows", [
     (11264, 2048, 97), (4100, 64, 300), (3001, 2112, 321), (900, 192, 1100), (5000, 16448, 260),
-    (2048, 4160, 210), (300, 11264, 701), (1100, 20544, 200)])
+    (2048, 4160, 210), (300, 11264, 701)])
 def test_tiles_match_oracle(device, fmt, out_width, in_width, rows):
     print(f"[gpu] tiles fmt={fmt} O={out_width} I={in_width} rows={rows}", flush=True)
     assert "qgemm_kernel" in native.gemv_kernel_name(fmt, out_width, in_width, rows)
