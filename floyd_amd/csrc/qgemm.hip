@@ -377,23 +377,6 @@ __device__ __forceinline__ void buffer_store_f32(__amdgpu_buffer_rsrc_t buf, flo
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), buf, voffset, 0, 0);
 }
 
-// silu(g) * u = g u / (1 + e^-g) in a third of the instructions of expf and an
-// IEEE division, to the same error (1.5 ulp): e^-g = 2^t with the rounding of
-// t = -g log2(e) carried into the result, the quotient by a reciprocal and one
-// remainder step.  g is held at -87 and above (silu there is under 2e-36), so
-// that e^-g and its reciprocal stay in fp32's normal range; NaN stays NaN.
-__device__ __forceinline__ float silu_times(float g, float u) {
-    constexpr float kLog2e = 1.44269504f, kLog2eRest = 1.92596299e-8f, kLn2 = 0.693147181f;
-    g = __builtin_elementwise_maximum(g, -87.0f);
-    const float t = -g * kLog2e;
-    const float rest = fmaf(-g, kLog2eRest, fmaf(-g, kLog2e, -t));
-    const float p = __builtin_amdgcn_exp2f(t);
-    const float d = 1.0f + fmaf(p, rest * kLn2, p);
-    const float r = __builtin_amdgcn_rcpf(d), n = g * u;
-    const float q = n * r;
-    return fmaf(fmaf(-d, q, n), r, q);
-}
-
 // Shares of a split reduction (the library's own memory, static, per GPU:
 // launches of one GPU run in order on the library's one stream).  A share is
 // the exact integer sum of its tile's limb products, as a double (at most 2^53
@@ -746,7 +729,8 @@ __global__ __launch_bounds__((QgShape<FMT, BM, LIMBS>::kThreads),
 #pragma unroll
                 for (int f = 0; f < kF; ++f) {
                     float v = limb_sum(f, r) * s * sw[f];
-                    if (DUAL) v = silu_times(v, limb_sum(f + kF, r) * s * su[f]);
+                    // in this order: g u may leave fp32's range where silu(g) u does not
+                    if (DUAL) v = silu(v) * (limb_sum(f + kF, r) * s * su[f]);
                     if (kResid) v = res[q][f] + v;
                     buffer_store_f32(y_buf, v, ycol[f] + row);
                 }
