@@ -260,7 +260,8 @@ int gemv_rows_per_block(const GemvPlan &plan, bool dual) {
 }
 
 bool gemv_mfma(const GemvParams &p, hipStream_t stream, std::string *name = nullptr);  // gemv_mfma.hip
-bool gemv_batch(const GemvParams &p, hipStream_t stream, std::string *name = nullptr);  // gemv_batch.hip
+bool gemv_batch(const GemvParams &p, bool fp32x, hipStream_t stream,
+                std::string *name = nullptr);  // gemv_batch.hip
 bool gemv_f32_batch(const GemvParams &p, hipStream_t stream,
                     std::string *name = nullptr);  // gemv_f32_batch.hip
 
@@ -274,11 +275,18 @@ static bool vector_takes(const GemvParams &p) {
            (!p.norm_w || aligned16(p.norm_w));
 }
 
-// One token row that the matrix-core kernels of gemv_mfma.hip do not take
-// stays on the vector kernel where that can run (q8 2048 x 1408: 3.44 against
-// 3.62 us on the batch kernel; at 2 rows 4.53 against 3.75).
-static bool vector_first(const GemvParams &p, bool vector_ok) {
-    return p.fmt == kF32 || (p.rows == 1 && vector_ok);
+// Calls that stay off the batch kernel: f32 matrices; one token row where the
+// vector kernel can run (q8 2048 x 1408: 3.44 against 3.62 us on the batch
+// kernel; at 2 rows 4.53 against 3.75); and small matrices of one token row
+// where it cannot.  There the generic kernel's waves, one per output, and the
+// serial loop of each both grow with the matrix: 100 x 100 2.5 us against 3.1
+// (q8) and 3.9 (q4) on the batch kernel, 300 x 333 3.2 against 4.2 and 4.7, 3000
+// x 333 4.9 against 4.5 and 4.3 against 4.9, 1001 x 999 6.9 against 5.8 and 5.2
+// against 5.4, 2500 x 1777 13.1 against 8.9 and 12.5 against 10.0.
+static bool off_batch(const GemvParams &p, bool vector_ok) {
+    constexpr double kGenericMax = 1 << 28;
+    return p.fmt == kF32 ||
+           (p.rows == 1 && (vector_ok || (double)p.O * p.I * p.I <= kGenericMax));
 }
 
 // Template name of the kernel gemv() launches for this shape (aligned
@@ -292,9 +300,12 @@ std::string gemv_kernel_name(int fmt, int O, int I, int rows, bool dual) {
     q.epilogue = dual ? kEpiSiluDual : q.epilogue;
     std::string mfma;
     q.x_stride = I;
+    const bool vector_ok = vector_takes(q);
     if (gemv_mfma(q, nullptr, &mfma) || gemv_f32_batch(q, nullptr, &mfma) ||
-        (q.rows > 4 && !gemv_batch_fits(q) && gemv_tiles(q, nullptr, &mfma)) || (!vector_first(q, vector_takes(q)) && gemv_batch(q, nullptr, &mfma)))
+        (vector_ok && q.rows > 4 && !gemv_batch_fits(q) && gemv_tiles(q, nullptr, &mfma)) ||
+        (!off_batch(q, vector_ok) && gemv_batch(q, !vector_ok, nullptr, &mfma)))
         return mfma;
+    if (!vector_ok) return "mlh::gemv_generic_kernel";
     const GemvPlan pl = plan_gemv(fmt, O, I, rows < kMaxGemvRows ? rows : kMaxGemvRows, dual);
     char buf[96];
     snprintf(buf, sizeof(buf), "mlh::gemv_kernel<0, %d, %d, %d, %d, %d, %d, %d>", fmt, pl.b,
@@ -319,10 +330,11 @@ int gemv(const GemvParams &p_in, hipStream_t stream) {
     if (gemv_mfma(p_in, stream) || gemv_f32_batch(p_in, stream))
         return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
     if (p_in.router_parts) return kErrArgs;
-    if (p_in.rows > 4 && !gemv_batch_fits(p_in) && gemv_tiles(p_in, stream))
-        return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+    // calls that the vector kernel does not take hold x in fp32 on every path
     const bool vector_ok = vector_takes(p_in);
-    if (!vector_first(p_in, vector_ok) && gemv_batch(p_in, stream))
+    if (vector_ok && p_in.rows > 4 && !gemv_batch_fits(p_in) && gemv_tiles(p_in, stream))
+        return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+    if (!off_batch(p_in, vector_ok) && gemv_batch(p_in, !vector_ok, stream))
         return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
     // token rows beyond 4 run as slices of 4 (register budget) along grid.y
     // of one launch

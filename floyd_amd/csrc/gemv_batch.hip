@@ -30,10 +30,21 @@
 // replays over rotating weights, before and after: q8 3072 x 2048 at 6 rows
 // 10.5 -> 5.0 us, at 64 rows 61.7 -> 10.4; q4 11264 x 2048 at 6 rows 15.8 ->
 // 7.4, at 16 rows 30.1 -> 10.1; q8 2048 x 11264 at 3 rows 60.8 -> 9.5, at 16
-// rows 278 -> 15.9; q8 1001 x 999 at 16 rows 14.9 -> 7.3.
+// rows 278 -> 15.9.
 //
-// Widths that are no multiple of 16 columns (q8) or 32 (q4) are cut there:
-// the rest of a row, under 32 products, is added in fp32 in the epilogue.
+// FP32X: the calls that the vector kernel does not take (ragged widths,
+// unaligned operands, rows past its LDS) keep x in fp32, as the kernel that
+// takes them otherwise (gemv.hip, gemv_generic_kernel) does: a range's step
+// would hold the columns far below its largest in few bits, which shows in the
+// outputs whose weight at the largest is small (999 columns, one of them 1e5
+// times the rest, weight 0: 3.5e-5 against 1e-7).  The products then run on
+// v_mfma_f32_16x16x4_f32, each started from zero and added pairwise, so a sum's
+// chain is no longer than the other kernel's (error against 64 bits, 11999 x
+// 11999 2.5e-7 there, 1.3e-7 here).  Widths that are no multiple of 16 columns
+// (q8) or 32 (q4) are cut there: the rest of a row, under 32 products, is added
+// in the epilogue.  Bound: the fp32 matrix units and the loads' latency; generic
+// kernel against this one, q8: 1001 x 999 at 6 rows 9.8 / 6.0 us, at 200 rows
+// 120 / 18; 11999 x 11999 at 1 row 189 / 126, at 16 rows 1769 / 143.
 #include "limb_split.h"
 
 #include <cstdio>
@@ -66,15 +77,10 @@ struct BatchGeom {
     int k_main = 0;  // columns that the matrix cores take
 };
 
-// 16 bytes of weights or x, at any address when UNAL.
-template <bool UNAL>
-__device__ __forceinline__ u32x4 load16_any(const uint8_t *p) {
-    if constexpr (!UNAL) {
-        return load_global16(p);
-    } else {
-        typedef unsigned u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
-        return *(const __attribute__((address_space(1))) u32x4_any *)p;
-    }
+// 16 bytes at any address.
+__device__ __forceinline__ u32x4 load16_any(const void *p) {
+    typedef unsigned u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+    return *(const __attribute__((address_space(1))) u32x4_any *)p;
 }
 
 // 16 packed nibbles (two words) as signed int8 in column order.
@@ -118,7 +124,94 @@ __device__ __forceinline__ float weight_at(const uint8_t *row, int k) {
     return (float)((k & 1) ? (b >> 4) - 8 : (b & 15) - 8);
 }
 
-template <int FMT, bool DUAL, int NB, int TOK, bool UNAL>
+// A wave's sums over a chunk in fp32: sum[b][r] += token row 4 g + r times weight
+// block b, and with a norm ss += x^2 of this lane's columns.  The wave takes
+// every kBtWaves-th piece of 64 columns (q8) or 128 (q4), so that a short row is
+// spread over the waves; lane (g, n) supplies the same 16 or 32 consecutive
+// columns of a piece for token row n and for weight row n.
+template <int FMT, int NB>
+__device__ __forceinline__ void chunk_f32(const float *xrow, const float *norm_w,
+                                          const uint8_t *const (&wrow)[NB], int chunk, int wave,
+                                          int k_main, int g, float (&sum)[NB][4], float &ss) {
+    typedef float f32x4v __attribute__((ext_vector_type(4)));
+    constexpr int kPieces = FMT == kQ8 ? 4 : 2, kCols = 64 / kPieces, kQuads = kCols / 4;
+    u32x4 x[kPieces][kQuads], nw[kPieces][kQuads] = {}, w[kPieces][NB];
+    int first[kPieces];  // column of the piece
+    bool in[kPieces];    // this lane's columns lie inside the row
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+        first[i] = ((chunk * kPieces + i) * kBtWaves + wave) * (4 * kCols);
+        if (first[i] >= k_main) break;  // uniform; the later pieces lie further on
+        int at = first[i] + kCols * g;
+        in[i] = at < k_main;
+        if (!in[i]) at = 0;  // x is taken as zero there
+#pragma unroll
+        for (int j = 0; j < kQuads; ++j) {
+            x[i][j] = load16_any(xrow + at + 4 * j);
+            if (norm_w) nw[i][j] = load16_any(norm_w + at + 4 * j);
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) w[i][b] = load16_any(wrow[b] + (FMT == kQ8 ? at : at / 2));
+    }
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+        if (first[i] >= k_main) break;
+        f32x4v part[kQuads / 4][NB];
+#pragma unroll
+        for (int h = 0; h < kQuads / 4; ++h) {
+            f32x4v quad[4][NB];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int q = 4 * h + j;
+                const u32x4 xq = x[i][q], nq = nw[i][q];
+                float v[4] = {__uint_as_float(xq.x), __uint_as_float(xq.y), __uint_as_float(xq.z),
+                              __uint_as_float(xq.w)};
+                const float n4[4] = {__uint_as_float(nq.x), __uint_as_float(nq.y),
+                                     __uint_as_float(nq.z), __uint_as_float(nq.w)};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    v[e] = in[i] ? v[e] : 0.0f;
+                    if (norm_w) {
+                        ss = fmaf(v[e], v[e], ss);
+                        v[e] = in[i] ? v[e] * n4[e] : 0.0f;
+                    }
+                }
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    const u32x4 d = w[i][b];
+                    const int word = FMT == kQ8 ? q : q / 2;  // of the four columns' weights
+                    const unsigned bits = word == 0 ? d.x : word == 1 ? d.y : word == 2 ? d.z : d.w;
+                    f32x4v m[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float wv = FMT == kQ8
+                                             ? (float)(int8_t)(bits >> (8 * e))
+                                             : (float)((int)((bits >> (16 * (q & 1) + 4 * e)) & 15) - 8);
+                        m[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], wv, f32x4v{0.f, 0.f, 0.f, 0.f},
+                                                                    0, 0, 0);
+                    }
+                    quad[j][b] = (m[0] + m[1]) + (m[2] + m[3]);
+                }
+                // the next products after these sums: 4 NB results in
+                // registers, not all of the piece's
+                if (q + 1 < kQuads) {
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) asm("" : "+v"(quad[j][b]), "+v"(x[i][q + 1]));
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+                part[h][b] = (quad[0][b] + quad[1][b]) + (quad[2][b] + quad[3][b]);
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                sum[b][r] += kQuads == 8 ? part[0][b][r] + part[kQuads / 4 - 1][b][r] : part[0][b][r];
+    }
+}
+
+template <int FMT, bool DUAL, int NB, int TOK, bool FP32X>
 __global__ __launch_bounds__(kBtThreads) void gemv_batch_kernel(GemvParams p, BatchGeom q) {
     constexpr int NR = 16 * NB;              // weight rows
     constexpr int NO = DUAL ? NR / 2 : NR;   // output columns
@@ -127,6 +220,7 @@ __global__ __launch_bounds__(kBtThreads) void gemv_batch_kernel(GemvParams p, Ba
     constexpr int kSubs = 16 / TOK;          // parts of a range over the lanes of a token row
     constexpr int SS = S / kSubs;            // steps per part
     static_assert(!DUAL || NB % 2 == 0, "gate and up blocks");
+    static_assert(!FP32X || TOK == 16, "a token row per lane of a lane row");
     static_assert(TOK * NR <= kBtPartFloats && TOK % 4 == 0, "share size; a C row group in one part");
     __shared__ __attribute__((aligned(16))) float red[kBtWaves][16][NR];
     __shared__ float red_ss[kBtWaves][16];
@@ -151,6 +245,10 @@ __global__ __launch_bounds__(kBtThreads) void gemv_batch_kernel(GemvParams p, Ba
         for (int r = 0; r < 4; ++r) sum[b][r] = 0.0f;
 
     for (int c = split; c < q.chunks; c += q.splits) {
+        if constexpr (FP32X) {
+            chunk_f32<FMT, NB>(xrow, p.norm_w, wrow, c, wave, q.k_main, g, sum, ss);
+            continue;
+        }
         const int base = (c * kBtWaves + wave) * kBtRange;
         if (base >= q.k_main) break;  // this wave's later chunks lie past the end too
         const bool whole = base + kBtRange <= q.k_main;
@@ -165,8 +263,7 @@ __global__ __launch_bounds__(kBtThreads) void gemv_batch_kernel(GemvParams p, Ba
             const int s = sub * SS + i / 4;
             col[i] = base + 16 * (FMT == kQ8 ? 4 * s + i % 4
                                              : 8 * (s >> 1) + 2 * (i % 4) + (s & 1));
-            const u32x4 d = load16_any<UNAL>(reinterpret_cast<const uint8_t *>(
-                xrow + (col[i] < q.k_main ? col[i] : 0) + 4 * g));
+            const u32x4 d = load_global16(xrow + (col[i] < q.k_main ? col[i] : 0) + 4 * g);
             v[i][0] = __uint_as_float(d.x);
             v[i][1] = __uint_as_float(d.y);
             v[i][2] = __uint_as_float(d.z);
@@ -176,8 +273,7 @@ __global__ __launch_bounds__(kBtThreads) void gemv_batch_kernel(GemvParams p, Ba
         if (has_norm) {
 #pragma unroll
             for (int i = 0; i < 4 * SS; ++i)
-                nw[i] = load16_any<UNAL>(reinterpret_cast<const uint8_t *>(
-                    p.norm_w + (col[i] < q.k_main ? col[i] : 0) + 4 * g));
+                nw[i] = load_global16(p.norm_w + (col[i] < q.k_main ? col[i] : 0) + 4 * g);
         }
         // weights: first column of this lane's 16 at step s (q4: a 16-byte
         // piece holds the lane's columns of two steps); column 0 past the end,
@@ -193,7 +289,7 @@ __global__ __launch_bounds__(kBtThreads) void gemv_batch_kernel(GemvParams p, Ba
         for (int b = 0; b < NB; ++b)
 #pragma unroll
             for (int i = 0; i < NW; ++i)
-                w[b][i] = load16_any<UNAL>(wrow[b] + (FMT == kQ8 ? at[i] : at[i] / 2));
+                w[b][i] = load_global16(wrow[b] + (FMT == kQ8 ? at[i] : at[i] / 2));
         if (!whole) {
 #pragma unroll
             for (int i = 0; i < 4 * SS; ++i)
@@ -296,17 +392,33 @@ __global__ __launch_bounds__(kBtThreads) void gemv_batch_kernel(GemvParams p, Ba
     auto finish = [&](int t, int j, float v, float u, float tss) {
         const int row = t0 + t, o = rb * NO + j;
         if (row >= p.rows || o >= p.O) return;
-        if (UNAL && q.k_main < p.I) {
+        if (FP32X && q.k_main < p.I) {
+            // eight columns' loads at a time
+            float vt = 0.0f, ut = 0.0f;
             const float *x = p.x + (long)row * p.x_stride;
             const uint8_t *wr = p.w + (long)o * row_bytes;
-            const uint8_t *ur = DUAL ? p.w2 + (long)o * row_bytes : nullptr;
-            for (int k = q.k_main; k < p.I; ++k) {
-                const float xv = x[k];
-                tss = fmaf(xv, xv, tss);
-                const float xn = has_norm ? xv * p.norm_w[k] : xv;
-                v = fmaf(xn, weight_at<FMT>(wr, k), v);
-                if (DUAL) u = fmaf(xn, weight_at<FMT>(ur, k), u);
+            const uint8_t *ur = DUAL ? p.w2 + (long)o * row_bytes : wr;
+            for (int k0 = q.k_main; k0 < p.I; k0 += 8) {
+                float xv[8], nv[8], wv[8], uv[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int k = min(k0 + e, p.I - 1);
+                    xv[e] = x[k];
+                    nv[e] = has_norm ? p.norm_w[k] : 1.0f;
+                    wv[e] = weight_at<FMT>(wr, k);
+                    uv[e] = DUAL ? weight_at<FMT>(ur, k) : 0.0f;
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    if (k0 + e >= p.I) break;
+                    tss = fmaf(xv[e], xv[e], tss);
+                    const float xn = xv[e] * nv[e];
+                    vt = fmaf(xn, wv[e], vt);
+                    if (DUAL) ut = fmaf(xn, uv[e], ut);
+                }
             }
+            v += vt;
+            u += ut;
         }
         const float inv = has_norm ? 1.0f / sqrtf(tss / (float)p.I + p.eps) : 1.0f;
         float out = v * inv * p.s[o];
@@ -372,7 +484,7 @@ __global__ __launch_bounds__(kBtThreads) void gemv_batch_kernel(GemvParams p, Ba
 
 struct BatchPlan {
     int nb = 2, tok = 16;
-    bool unal = false;
+    bool fp32x = false;
     BatchGeom geom;
     dim3 grid;
 };
@@ -387,23 +499,21 @@ struct BatchPlan {
 // us; 52.9 when split up to 512).
 constexpr int kBtTarget = kBtMaxParts;
 
-BatchPlan plan_batch(const GemvParams &p, bool unal) {
+BatchPlan plan_batch(const GemvParams &p, bool fp32x) {
     BatchPlan pl;
     const bool dual = p.epilogue == kEpiSiluDual;
     const int cut = p.fmt == kQ8 ? 16 : 32;
-    pl.unal = unal;
+    pl.fp32x = fp32x;
     pl.geom.k_main = p.I / cut * cut;
     pl.geom.chunks = (pl.geom.k_main + kBtChunk - 1) / kBtChunk;
-    pl.tok = p.rows <= 4 ? 4 : p.rows <= 8 ? 8 : 16;
+    pl.tok = fp32x || p.rows > 8 ? 16 : p.rows > 4 ? 8 : 4;
     const int groups = (p.rows + pl.tok - 1) / pl.tok;
     const long weight_rows = (long)p.O * (dual ? 2 : 1);
     auto blocks = [&](int nb) { return (int)((weight_rows + 16 * nb - 1) / (16 * nb)); };
     auto units = [&](int nb) { return (long)blocks(nb) * groups * pl.geom.chunks; };
     pl.nb = 2;
-    if (!unal) {
-        if (!dual && (pl.tok == 4 || units(1) <= kBtTarget)) pl.nb = 1;
-        else if (pl.tok >= 8 && units(2) > kBtTarget) pl.nb = 4;
-    }
+    if (!dual && (pl.tok == 4 || units(1) <= kBtTarget)) pl.nb = 1;
+    else if (!fp32x && pl.tok >= 8 && units(2) > kBtTarget) pl.nb = 4;
     const int n = blocks(pl.nb);
     int splits = 1;
     while (splits < pl.geom.chunks && splits < kBtMaxSplits &&
@@ -414,47 +524,49 @@ BatchPlan plan_batch(const GemvParams &p, bool unal) {
     return pl;
 }
 
-template <int FMT, bool DUAL, int NB, int TOK, bool UNAL>
+template <int FMT, bool DUAL, int NB, int TOK, bool FP32X = false>
 void launch(const GemvParams &p, const BatchPlan &pl, hipStream_t stream) {
-    hipLaunchKernelGGL((gemv_batch_kernel<FMT, DUAL, NB, TOK, UNAL>), pl.grid, dim3(kBtThreads), 0,
+    hipLaunchKernelGGL((gemv_batch_kernel<FMT, DUAL, NB, TOK, FP32X>), pl.grid, dim3(kBtThreads), 0,
                        stream, p, pl.geom);
 }
 template <int FMT, bool DUAL, int TOK>
 void launch_nb(const GemvParams &p, const BatchPlan &pl, hipStream_t stream) {
-    if (pl.unal) return launch<FMT, DUAL, 2, TOK, true>(p, pl, stream);
     if constexpr (!DUAL) {
-        if (pl.nb == 1) return launch<FMT, DUAL, 1, TOK, false>(p, pl, stream);
+        if (pl.nb == 1) return launch<FMT, DUAL, 1, TOK>(p, pl, stream);
     }
     if constexpr (TOK >= 8) {
-        if (pl.nb == 4) return launch<FMT, DUAL, 4, TOK, false>(p, pl, stream);
+        if (pl.nb == 4) return launch<FMT, DUAL, 4, TOK>(p, pl, stream);
     }
-    launch<FMT, DUAL, 2, TOK, false>(p, pl, stream);
+    launch<FMT, DUAL, 2, TOK>(p, pl, stream);
 }
 template <int FMT, bool DUAL>
 void launch_tok(const GemvParams &p, const BatchPlan &pl, hipStream_t stream) {
-    if (pl.tok == 4) launch_nb<FMT, DUAL, 4>(p, pl, stream);
+    if (pl.fp32x) {
+        if constexpr (!DUAL) {
+            if (pl.nb == 1) return launch<FMT, DUAL, 1, 16, true>(p, pl, stream);
+        }
+        launch<FMT, DUAL, 2, 16, true>(p, pl, stream);
+    } else if (pl.tok == 4) launch_nb<FMT, DUAL, 4>(p, pl, stream);
     else if (pl.tok == 8) launch_nb<FMT, DUAL, 8>(p, pl, stream);
     else launch_nb<FMT, DUAL, 16>(p, pl, stream);
 }
 
 }  // namespace
 
-// Launches the kernel for p (q8 / q4, no pre-split x, no router partials);
-// false, launching nothing, when it does not take it.  With `name` set it
+// Launches the kernel for p (q8 / q4, no pre-split x, no router partials), with
+// x in fp32 (FP32X) or, where the vector kernel takes p, in limbs; false,
+// launching nothing, when it does not take it.  With `name` set it
 // launches nothing and stores the kernel's template name.
-bool gemv_batch(const GemvParams &p, hipStream_t stream, std::string *name) {
+bool gemv_batch(const GemvParams &p, bool fp32x, hipStream_t stream, std::string *name) {
     if ((p.fmt != kQ8 && p.fmt != kQ4) || p.limbs || p.router_parts) return false;
-    auto al = [](const void *q) { return ((uintptr_t)q & 15u) == 0; };
     const bool dual = p.epilogue == kEpiSiluDual;
-    const bool unal = p.I % (p.fmt == kQ8 ? 16 : 32) != 0 || !al(p.w) || (dual && !al(p.w2)) ||
-                      !al(p.x) || p.x_stride % 4 || (p.norm_w && !al(p.norm_w));
-    const BatchPlan pl = plan_batch(p, unal);
+    const BatchPlan pl = plan_batch(p, fp32x);
     if (pl.grid.z > 65535) return false;
     if (name) {
         char buf[96];
         snprintf(buf, sizeof(buf),
                  "mlh::(anonymous namespace)::gemv_batch_kernel<%d, %s, %d, %d, %s>", p.fmt,
-                 dual ? "true" : "false", pl.nb, pl.tok, pl.unal ? "true" : "false");
+                 dual ? "true" : "false", pl.nb, pl.tok, pl.fp32x ? "true" : "false");
         *name = buf;
         return true;
     }

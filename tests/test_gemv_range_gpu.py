@@ -4,8 +4,11 @@ import numpy as np
 import pytest
 
 import oracle_lib as O
+from conftest import rel_l2
 from floyd_amd import native
 from floyd_amd.native import DeviceBuffer
+from test_gemv_batch_gpu import shifted
+from test_gemv_gpu import make_weights
 
 pytestmark = pytest.mark.gpu
 
@@ -46,3 +49,98 @@ def test_swiglu_over_the_range_of_fp32(device, fmt, rows, kernel):
         np.testing.assert_array_equal(got[r][~ordinary], expect[~ordinary])
         # results below fp32's normal range count as zero
         np.testing.assert_allclose(got[r][ordinary], expect[ordinary], rtol=1e-6, atol=1.2e-38)
+
+
+def unpacked(fmt, q, in_width):
+    """The stored integers [out, in] in 64 bits."""
+    if fmt == 1:
+        return q.view(np.int8).astype(np.float64)
+    return (np.stack([q & 15, q >> 4], 2).reshape(q.shape[0], -1)[:, :in_width]).astype(np.float64) - 8
+
+
+def store(fmt, q, column, value):
+    """Sets one column of packed weights."""
+    if fmt == 1:
+        q.view(np.int8)[:, column] = value
+    elif column % 2:
+        q[:, column // 2] = q[:, column // 2] & 15 | (value + 8) << 4
+    else:
+        q[:, column // 2] = q[:, column // 2] & 240 | (value + 8)
+
+
+def normed(x, nw):
+    x = x.astype(np.float64)
+    return x / np.sqrt((x * x).mean(1, keepdims=True) + 1e-5) * nw
+
+
+# (out, in, rows, byte offset of w, of x): widths that are no multiple of a
+# 16-byte weight chunk, operands at any address, rows wider than the vector
+# kernel's LDS
+@pytest.mark.parametrize("fmt", [1, 2])
+@pytest.mark.parametrize("out_width,in_width,rows,w_off,x_off", [
+    (50, 999, 1, 0, 0), (2000, 999, 1, 0, 0), (50, 999, 6, 0, 0), (333, 4111, 40, 0, 0), (70, 95, 17, 0, 0),
+    (60, 40, 3, 0, 0), (40, 15, 2, 0, 0), (3, 2113, 700, 0, 0), (70, 2112, 1, 1, 0),
+    (70, 2112, 20, 0, 4), (1500, 2112, 900, 3, 12), (40, 45056, 6, 0, 0), (4096, 45056, 70, 0, 0)])
+def test_small_columns_beside_large_ones_keep_fp32(device, fmt, out_width, in_width, rows, w_off,
+                                                   x_off):
+    """Calls outside the vector kernel's shapes hold x in fp32: columns 1e5 times
+    the rest whose weights are 0 take nothing from the others' precision.
+
+    Tolerance: fp32 roundings of products, norm and sums that are added pairwise,
+    about 25 of them one after the other at the widest row, 2^-24 each and none
+    larger than the result's rms times a few: 1e-6.
+    """
+    print(f"[gpu] large columns fmt={fmt} O={out_width} I={in_width} rows={rows} "
+          f"+{w_off} +{x_off}", flush=True)
+    if not (w_off or x_off):
+        name = native.gemv_kernel_name(fmt, out_width, in_width, rows)
+        assert "gemv_generic" in name or "gemv_batch_kernel" in name and name.endswith("true>")
+    q, s = make_weights(fmt, out_width, in_width, seed=out_width + in_width)
+    q = q.reshape(out_width, -1)
+    x = O.fill_normal(rows * in_width, 7 + rows).reshape(rows, in_width)
+    for c in {3, in_width // 2, in_width - 1}:
+        x[:, c] *= 1e5
+        store(fmt, q, c, 0)
+    nw = O.fill_normal(in_width, 4, mean=1.0, std=0.1)
+    ds, dn = DeviceBuffer.from_array(s), DeviceBuffer.from_array(nw)
+    dy = DeviceBuffer(rows * out_width * 4)
+    keep_w, w = shifted(q, w_off)
+    keep_x, xp = shifted(x, x_off)
+    wt = (unpacked(fmt, q, in_width) * s.astype(np.float64)[:, None]).T
+    for norm in (None, dn):
+        native.gemv(fmt, w, ds, xp, dy, out_width, in_width, rows, norm_w=norm, eps=1e-5)
+        expect = (normed(x, nw) if norm else x.astype(np.float64)) @ wt
+        assert rel_l2(dy.download(np.float32).reshape(rows, out_width), expect) < 1e-6
+    native.gemv_swiglu(fmt, w, ds, w, ds, xp, dy, out_width, in_width, rows, norm_w=dn, eps=1e-5)
+    g = normed(x, nw) @ wt
+    # silu(g) g moves by up to 2.1 |g| of g's error, and g here is small
+    assert rel_l2(dy.download(np.float32).reshape(rows, out_width), g / (1 + np.exp(-g)) * g) < 4e-6
+
+
+@pytest.mark.parametrize("fmt", [1, 2])
+@pytest.mark.parametrize("out_width,in_width,rows", [
+    (100, 2048, 3), (100, 2080, 7), (64, 6144, 40), (2048, 4160, 210), (11264, 2048, 130)])
+def test_limbs_hold_30_bits_of_the_largest(device, fmt, out_width, in_width, rows):
+    """The limb kernels (the batch kernel in all its token tiles, the GEMM tiles
+    whole and split) on rows with columns 1e4 times the rest.
+
+    Bound of one output: an element is cut by less than 2^-29 of the row's
+    largest, so its sum by that times the sum of its weights' magnitudes; the
+    integer sums are exact, their conversions and the at most 30 additions of
+    ranges round 2^-24 of the sum of the products' magnitudes each.
+    """
+    print(f"[gpu] limbs fmt={fmt} O={out_width} I={in_width} rows={rows}", flush=True)
+    name = native.gemv_kernel_name(fmt, out_width, in_width, rows)
+    assert "qgemm_kernel" in name or name.endswith("false>")
+    q, s = make_weights(fmt, out_width, in_width, seed=out_width + in_width)
+    q = q.reshape(out_width, -1)
+    x = O.fill_normal(rows * in_width, 7 + rows).reshape(rows, in_width)
+    x[:, ::301] *= 1e4
+    dw, ds, dx = (DeviceBuffer.from_array(a) for a in (q, s, x))
+    dy = DeviceBuffer(rows * out_width * 4)
+    native.gemv(fmt, dw, ds, dx, dy, out_width, in_width, rows)
+    wt = (unpacked(fmt, q, in_width) * s.astype(np.float64)[:, None]).T
+    x = x.astype(np.float64)
+    bound = 2.0 ** -29 * np.abs(x).max(1)[:, None] * np.abs(wt).sum(0) + \
+        32 * 2.0 ** -24 * (np.abs(x) @ np.abs(wt))
+    assert (np.abs(dy.download(np.float32).reshape(rows, out_width) - x @ wt) <= bound).all()
