@@ -300,6 +300,7 @@ std::string gemv_kernel_name(int fmt, int O, int I, int rows, bool dual) {
     q.epilogue = dual ? kEpiSiluDual : q.epilogue;
     std::string mfma;
     q.x_stride = I;
+    q.y_stride = O;
     const bool vector_ok = vector_takes(q);
     if (gemv_mfma(q, nullptr, &mfma) || gemv_f32_batch(q, nullptr, &mfma) ||
         (vector_ok && q.rows > 4 && !gemv_batch_fits(q) && gemv_tiles(q, nullptr, &mfma)) ||

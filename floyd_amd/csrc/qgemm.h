@@ -31,6 +31,11 @@ constexpr int kQgBW = 256;  // weight rows per tile
 constexpr int kQgBK = 64;   // k per pipeline stage
 constexpr int kQgGroup = 4; // row tiles per locality group
 constexpr int kQgMaxTasks = 272;
+// Outputs and residuals of a tile are addressed by 31-bit byte offsets from the
+// tile's first row (columns past the last get the largest one, which has to lie
+// outside the tile's rows): floats between rows are at most this many.
+constexpr long kQgOutside = 0x7FFFFFFFL;
+constexpr long kQgMaxStride = kQgOutside / (4 * kQgBM);
 
 // Quantised activations lie in blocks of 8 rows x 128 columns: the three limbs'
 // (hi, mid, lo) 8 x 128 bytes one after the other, a row block's column blocks

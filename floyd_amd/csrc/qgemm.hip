@@ -672,7 +672,7 @@ __global__ __launch_bounds__((QgShape<FMT, BM, LIMBS>::kThreads),
     // offset is set there.  Weight scales and residual rows are loaded before
     // the stores they precede: a wait for a load after a store waits for both.
     constexpr int kF = DUAL ? kNF / 2 : kNF;
-    constexpr unsigned kOutside = 0x7FFFFFFFu;
+    constexpr unsigned kOutside = (unsigned)kQgOutside;
     const int rows_here = min(tk.rows - m0, BM);
     float sw[kF], su[kF];
     unsigned ycol[kF], rcol[kF];
@@ -1071,6 +1071,7 @@ static int launch_qgemm_fmt(int fmt, bool dual, int kind, const QGemmLaunch &L, 
 int qgemm_single(int fmt, bool dual, const GemmTask &task, hipStream_t stream) {
     if (!qgemm_shape_ok(fmt, task.k) || task.rows <= 0 || task.n_out <= 0 || !task.w ||
         !task.s || !task.a || task.a_width < task.k || !task.a_scale || !task.y ||
+        task.y_stride > kQgMaxStride || (task.resid && task.resid_stride > kQgMaxStride) ||
         (dual && (!task.w2 || !task.s2)))
         return kErrArgs;
     QGemmLaunch L;
@@ -1176,7 +1177,8 @@ bool gemv_tiles(const GemvParams &p, hipStream_t stream, std::string *name) {
     const bool dual = p.epilogue == kEpiSiluDual;
     auto al = [](const void *v) { return ((uintptr_t)v & 15u) == 0; };
     if (!qgemm_shape_ok(p.fmt, p.I) || p.I > kTilesMaxWidth || p.limbs || p.router_parts || !al(p.w) ||
-        (dual && !al(p.w2)) || !al(p.x) || p.x_stride % 4 || (p.norm_w && !al(p.norm_w)))
+        (dual && !al(p.w2)) || !al(p.x) || p.x_stride % 4 || (p.norm_w && !al(p.norm_w)) ||
+        p.y_stride > kQgMaxStride || (p.resid && p.resid_stride > kQgMaxStride))
         return false;
     if (name) {
         char buf[64];

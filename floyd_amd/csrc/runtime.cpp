@@ -921,7 +921,8 @@ constexpr int kMoeGemmMinRows = 3;
 
 // out_w: weight rows of the launch (a SwiGLU pair: gate and up).
 bool use_gemm(const MoonlightSession *s, int fmt, int rows, int in_w, int out_w) {
-    if (rows < kGemmMinRows || !s->aq || in_w > s->aq_width || !qgemm_shape_ok(fmt, in_w))
+    if (rows < kGemmMinRows || !s->aq || in_w > s->aq_width || !qgemm_shape_ok(fmt, in_w) ||
+        out_w > kQgMaxStride)
         return false;
     return !gemv_batch_fits(out_w, rows, in_w);
 }

@@ -1,0 +1,43 @@
+"""Shapes at the ends of the int8 GEMM tiles' integer ranges (qgemm.h): byte
+offsets inside a tile, which the dispatch has to keep in range.  No GPU but for
+the test that runs the call."""
+import numpy as np
+import pytest
+
+from floyd_amd import native
+from floyd_amd.native import DeviceBuffer
+
+
+@pytest.mark.parametrize("fmt", [1, 2])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_tile_rows_stay_within_31_bit_offsets(fmt, swiglu):
+    """A tile addresses its output rows by 31-bit byte offsets from its first one:
+    64 rows of more than 2^23 floats (128 rows of the widest tile: 2^22) reach
+    past them, so such a matrix is left to the batch kernel."""
+    name = {o: native.gemv_kernel_name(fmt, o, 64, 64, swiglu)
+            for o in (4194303, 4194304, 8388700, 16777300)}
+    assert "qgemm_kernel" in name.pop(4194303)
+    assert all("gemv_batch_kernel" in n for n in name.values()), name
+
+
+@pytest.mark.gpu
+def test_outputs_of_over_2_gib(device):
+    """64 token rows of 8,388,700 outputs, every output against numpy's fp32
+    product (64 columns: at most 64 roundings of 2^-24 each of the sum of the
+    products' magnitudes)."""
+    out_width, in_width, rows = 8388700, 64, 64
+    print(f"[gpu] O={out_width} I={in_width} rows={rows}", flush=True)
+    rng = np.random.default_rng(3)
+    q = rng.integers(-127, 128, (out_width, in_width), dtype=np.int8)
+    s = np.full(out_width, 1.0 / 127, np.float32)
+    x = rng.standard_normal((rows, in_width)).astype(np.float32)
+    dq, ds, dx = (DeviceBuffer.from_array(a) for a in (q.view(np.uint8), s, x))
+    dy = DeviceBuffer(rows * out_width * 4)
+    native.gemv(1, dq, ds, dx, dy, out_width, in_width, rows)
+    step = 1 << 20
+    for r in (0, 31, 62, 63):
+        got = dy.download(np.float32, out_width, r * out_width * 4)
+        for o in range(0, out_width, step):
+            w = q[o:o + step].astype(np.float32)
+            bound = 64 * 2.0 ** -23 * (np.abs(w) @ np.abs(x[r])) / 127
+            assert (np.abs(got[o:o + step] - (w @ x[r]) / 127) <= bound).all(), (r, o)
