@@ -150,7 +150,12 @@ __host__ __device__ inline bool moe_shared_splits(int inter, int shared_width) {
 }
 int moe_gemm(const MoeGemmParams &p, hipStream_t stream);
 
+// Widest reduction whose int32 sums cannot overflow: a limb and a stored weight
+// (q4 on the LDS tiles: 16 times the weight) are at most 128 each.
+constexpr int kQgMaxK = 0x7FFFFFFF / (128 * 128) / kQgBK * kQgBK;
 // Shapes the MFMA path takes (k a multiple of kQgBK, 16-byte aligned rows).
-bool qgemm_shape_ok(int fmt, int k);
+inline bool qgemm_shape_ok(int fmt, int k) {
+    return (fmt == kQ8 || fmt == kQ4) && k > 0 && k <= kQgMaxK && k % kQgBK == 0;
+}
 
 }  // namespace mlh

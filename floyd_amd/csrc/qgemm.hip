@@ -37,10 +37,6 @@ typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr float kQuantMax = 4194304.0f;  // 2^22: |65536 * hi + 256 * mid + lo| bound
 
-bool qgemm_shape_ok(int fmt, int k) {
-    return (fmt == kQ8 || fmt == kQ4) && k > 0 && k % kQgBK == 0;
-}
-
 // ---------------------------------------------------------------------------
 // activation quantisation: one wave per row
 // ---------------------------------------------------------------------------
@@ -1092,7 +1088,8 @@ int qgemm_single(int fmt, bool dual, const GemmTask &task, hipStream_t stream) {
 // may be captured.)
 constexpr long kTilesBytes = 64L << 20;
 constexpr int kTilesRows = 8192;
-constexpr int kTilesMaxWidth = 65536;  // int32 sums: 2^14 per column
+constexpr int kTilesMaxWidth = 65536;  // the shares' doubles are exact to here
+static_assert(kTilesMaxWidth <= kQgMaxK, "int32 sums");
 __device__ int8_t tiles_limbs[kTilesBytes];
 __device__ float tiles_scale[kTilesRows];
 static std::mutex tiles_mutex;

@@ -1,11 +1,42 @@
 """Shapes at the ends of the int8 GEMM tiles' integer ranges (qgemm.h): byte
-offsets inside a tile, which the dispatch has to keep in range.  No GPU but for
-the test that runs the call."""
+offsets inside a tile and int32 sums, which the dispatch has to keep in range.
+No GPU but for the test that runs the call."""
+import os
+import shutil
+import subprocess
+
 import numpy as np
 import pytest
 
 from floyd_amd import native
 from floyd_amd.native import DeviceBuffer
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+
+
+def host_values(tmp_path, *expressions):
+    """Integer expressions over qgemm.h, evaluated by a host program."""
+    src, exe = tmp_path / "values.cpp", tmp_path / "values"
+    prints = "".join('printf("%%ld\\n", (long)(%s));' % e for e in expressions)
+    src.write_text('#include <cstdio>\n#include "qgemm.h"\n'
+                   "using namespace mlh;\nint main() { %s }\n" % prints)
+    subprocess.run([HIPCC, "-std=c++17", "--cuda-host-only", "-x", "hip",
+                    "-I" + os.path.join(ROOT, "floyd_amd", "csrc"),
+                    "-I" + os.path.join(ROOT, "include"), str(src), "-o", str(exe)],
+                   check=True, capture_output=True)
+    out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
+    return [int(v) for v in out.split()]
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+def test_reductions_stay_within_int32(tmp_path):
+    """A limb of -128 against a weight of -128 (q8, or 16 times a q4 weight of -8)
+    in every column adds up to 2^14 a column: 2^31 at 131072 columns."""
+    at = (64, 131008, 131072, 131136, 1 << 20)
+    got = host_values(tmp_path, *["qgemm_shape_ok(%s, %d)" % (f, k)
+                                  for f in ("kQ8", "kQ4") for k in at])
+    assert got == 2 * [int(k * 2 ** 14 < 2 ** 31) for k in at]
 
 
 @pytest.mark.parametrize("fmt", [1, 2])
