@@ -59,6 +59,12 @@ __host__ __device__ inline long limb_at(long row, int col, int width) {
            (col & 127);
 }
 
+// Tasks of gathered rows (a_rows) reach each from row 0 by a 32-bit byte offset;
+// offsets from kQgGatherBytes on read zeros.
+constexpr long kQgGatherBytes = 0xF0000000L;
+// Most token rows of one moe_gemm call, whose expert tasks gather them.
+inline long moe_gemm_max_rows(int hidden) { return kQgGatherBytes / limb_row_block(hidden) * 8; }
+
 // One independent product: rows x n_out outputs, reduction length k.
 struct GemmTask {
     const uint8_t *w = nullptr, *w2 = nullptr;  // [n_out][k] packed (w2: up rows, SwiGLU)

@@ -441,7 +441,7 @@ __global__ __launch_bounds__((QgShape<FMT, BM, LIMBS>::kThreads),
     const int w_ld = tk.w_ld ? tk.w_ld : tk.k;
     const long w_row_bytes = FMT == kQ8 ? w_ld : w_ld / 2;
     // the tile's first activation row block and weight row, in 64 bits: the
-    // offsets from there fit 32 (gathered rows are those of one routing call)
+    // offsets from there fit 32 (gathered rows: moe_gemm_max_rows)
     const int a_first = tk.a_rows ? 0 : (tk.a_row0 + m0) & ~7;
     const int8_t *const a_base = tk.a + limb_at<LIMBS>(a_first, 0, tk.a_width);
     const uint8_t *const w_base = tk.w + n0 * w_row_bytes;
@@ -469,7 +469,7 @@ __global__ __launch_bounds__((QgShape<FMT, BM, LIMBS>::kThreads),
     // so it loads the logical chunk (l % chunks) ^ g(row).  The limbs share a
     // lane's A rows.  Byte offsets of this lane's A rows; past the task's end
     // outside the buffer (read as zeros):
-    constexpr long kABytes = 0xF0000000L;
+    constexpr long kABytes = kQgGatherBytes;
     const int alr = lane >> 3, alc = lane & 7;
     unsigned a_off[Sh::kAOffs];
 #pragma unroll
@@ -1407,6 +1407,7 @@ __global__ __launch_bounds__(64 * kPrepWaves) void moe_prep_kernel(QuantSeg a, M
 
 int moe_gemm(const MoeGemmParams &p, hipStream_t stream) {
     if (p.rows <= 0 || p.experts <= 0 || p.experts + 2 > kQgMaxTasks || p.top_k <= 0 ||
+        p.rows > moe_gemm_max_rows(p.hidden) ||
         !qgemm_shape_ok(p.expert_fmt, p.hidden) || !qgemm_shape_ok(p.expert_fmt, p.inter) ||
         (p.has_shared && (!qgemm_shape_ok(p.shared_fmt, p.hidden) ||
                           !qgemm_shape_ok(p.shared_fmt, p.shared_width))))

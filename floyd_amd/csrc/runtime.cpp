@@ -1339,10 +1339,11 @@ int experts(MoonlightSession *s, int layer, const float *x, int rows, const floa
 }
 
 // Token rows of one routing call: each routes at most kRouteMaxPositions
-// (row, slot) positions (the route-table kernels keep them in LDS).
+// (row, slot) positions (the route-table kernels keep them in LDS), and the GEMM
+// tiles reach at most moe_gemm_max_rows (fewer than 16384 from 81,921 columns on).
 int moe_chunk_rows(const ModelConfig &c) {
     const int k = c.experts_per_token > 0 ? c.experts_per_token : 1;
-    return kRouteMaxPositions / k;
+    return (int)std::min<long>(kRouteMaxPositions / k, moe_gemm_max_rows(c.hidden_size));
 }
 
 // The kernels of one forward over `count` token rows at `start` (embed,

@@ -39,6 +39,21 @@ def test_reductions_stay_within_int32(tmp_path):
     assert got == 2 * [int(k * 2 ** 14 < 2 ** 31) for k in at]
 
 
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+def test_gathered_rows_stay_within_32_bit_offsets(tmp_path):
+    """The MoE tiles reach a gathered row's limbs by a 32-bit offset from row 0,
+    of which kQgGatherBytes and more mean a row that is not there: the largest
+    batch's last row ends below, and ordinary batches are not cut (16384 rows
+    route at most)."""
+    widths = (64, 2048, 7168, 16384, 81920, 81984, 131008)
+    rows = host_values(tmp_path, *["moe_gemm_max_rows(%d)" % w for w in widths])
+    ends = host_values(tmp_path, "kQgGatherBytes", *["limb_bytes(moe_gemm_max_rows(%d), %d)" % (w, w)
+                                                     for w in widths])
+    assert ends[0] + 16 * 1024 * 1024 < 2 ** 32  # and a slice's offset on top
+    assert all(e <= ends[0] for e in ends[1:])
+    assert [r >= 16384 for r in rows] == [w <= 81920 for w in widths] and min(rows) > 8192
+
+
 @pytest.mark.parametrize("fmt", [1, 2])
 @pytest.mark.parametrize("swiglu", [False, True])
 def test_tile_rows_stay_within_31_bit_offsets(fmt, swiglu):
