@@ -24,7 +24,6 @@ namespace {
 
 constexpr int kFbWaves = 8;
 constexpr int kFbThreads = 64 * kFbWaves;
-constexpr long kFbMaxLds = 144 * 1024;  // token rows of a workgroup
 
 template <int B> struct FbShape {
     static constexpr int kR = B <= 8 ? 8 : 4;          // weight rows per wave and pass
@@ -124,7 +123,7 @@ void launch(const GemvParams &p, hipStream_t stream) {
     static const bool attr = [] {
         return hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_f32_batch_kernel<B>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)kFbMaxLds) == hipSuccess;
+                                   (int)kF32BatchLds) == hipSuccess;
     }();
     (void)attr;
     // as many workgroups as fit the CUs at once, twice over, so that the token
@@ -140,27 +139,15 @@ void launch(const GemvParams &p, hipStream_t stream) {
 }  // namespace
 
 // Launches the kernel for p; false, launching nothing, where it does not take p
-// or the vector kernel is as fast.  With `name` set it launches nothing and
-// stores the kernel's template name.
-// With a norm it wins from 3 token rows and 4096 weight rows, without one from
-// 5 (one pass of the vector kernel holds 4) and 8192.  Measured on MI355X,
-// vector kernel against this one, with norm: 163840 x 2048 at 2 rows 231 / 211
-// us, 3 rows 384 / 212, 8 rows 838 / 214, 16 rows 1673 / 327; 10000 x 2048 at 3
-// rows 29.6 / 18.0; 4100 x 2048 at 3 rows 16.1 / 15.8, at 2 rows 10.2 / 14.4;
-// 20000 x 5120 at 4 rows 129 / 85.  Without: 163840 x 2048 at 4 rows 224 / 212,
-// at 6 rows 423 / 212; 10000 x 2048 at 4 rows 16.3 / 17.8, at 6 rows 26.5 /
-// 20.6; 4100 x 2048 at 6 rows 13.9 / 18.7.
+// or the vector kernel is as fast (f32_batch_rows).  With `name` set it launches
+// nothing and stores the kernel's template name.
 bool gemv_f32_batch(const GemvParams &p, hipStream_t stream, std::string *name) {
     auto al = [](const void *q) { return ((uintptr_t)q & 15u) == 0; };
-    if (p.fmt != kF32 || p.rows < (p.norm_w ? 3 : 5) || p.O < (p.norm_w ? 4096 : 8192) ||
-        p.epilogue == kEpiSiluDual || p.limbs || p.router_parts || p.I % 4 || !al(p.w) || !al(p.x) ||
-        p.x_stride % 4 || (p.norm_w && !al(p.norm_w)))
+    if (p.fmt != kF32 || p.epilogue == kEpiSiluDual || p.limbs || p.router_parts || p.I % 4 ||
+        !al(p.w) || !al(p.x) || p.x_stride % 4 || (p.norm_w && !al(p.norm_w)))
         return false;
-    // token rows of a workgroup, halved until they fit the LDS; of two passes
-    // the vector kernel's are as fast (20000 x 5120 at 6 rows 125 / 139 us)
-    int b = p.rows <= 4 ? 4 : p.rows <= 8 ? 8 : 16;
-    while (b > 4 && (long)b * p.I * 4 > kFbMaxLds) b /= 2;
-    if ((long)b * p.I * 4 > kFbMaxLds || (!p.norm_w && b < 8) || (p.rows + b - 1) / b > 65535) return false;
+    const int b = f32_batch_rows(p.O, p.I, p.rows, p.norm_w != nullptr);
+    if (!b || (p.rows + b - 1) / b > 65535) return false;
     if (name) {
         char buf[80];
         snprintf(buf, sizeof(buf), "mlh::(anonymous namespace)::gemv_f32_batch_kernel<%d>", b);

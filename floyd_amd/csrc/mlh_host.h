@@ -80,6 +80,38 @@ inline bool gemv_batch_fits(const GemvParams &p) {
         return gemv_batch_fits((long)p.O * (p.epilogue == kEpiSiluDual ? 2 : 1), p.rows, p.I);
     return ((long)p.O + 63) / 64 * ((p.rows + 15) / 16) * chunks <= 600 + 110 * chunks;
 }
+// Token rows of a workgroup of the f32 batch kernel (gemv_f32_batch.hip: a
+// workgroup holds them in LDS) for a matrix of `weight_rows` rows: 4, 8 or 16,
+// halved until they fit; 0 where the vector kernel, which takes 4 token rows a
+// pass, is as fast.  A wave's pass over its few weight rows costs some 4 us of
+// reductions and latency whatever their length, so narrow matrices stay off it.
+// With a norm, which the vector kernel applies again for each of its weight
+// rows, the line is 352 columns, and 8192 over the token rows of a 16-row
+// workgroup (their padding is multiplied too); without one 1024 columns and at
+// least 5 token rows, and with 16-row workgroups either all of their passes of 4
+// or two full rounds of workgroups over the CUs.  Measured on MI355X, this kernel
+// against the vector kernel, with norm: 163840 x 2048 at 2 rows 211 / 231 us, 3
+// rows 212 / 384, 8 rows 214 / 838, 16 rows 327 / 1673; 9000 x 352 at 4 rows 8 / 9,
+// at 9 rows 24 / 17; 9000 x 1024 at 9 rows 32 / 33; 20000 x 256 at 3 rows 13 / 9;
+// 70000 x 64 at 16 rows 49 / 27; 4100 x 2048 at 3 rows 15.8 / 16.1.  Without:
+// 163840 x 2048 at 4 rows 212 / 224, at 6 rows 212 / 423; 20000 x 704 at 8 rows 25 /
+// 21, 20000 x 1024 29 / 33; 9000 x 2048 at 9 rows 45 / 36, at 16 rows 45 / 49; 20000 x
+// 1024 at 9 rows 45 / 46; 20000 x 5120 at 6 rows (two workgroups of 4) 139 / 125;
+// 4100 x 2048 at 6 rows 18.7 / 13.9.
+constexpr long kF32BatchLds = 144 * 1024;
+inline int f32_batch_rows(long weight_rows, int in_width, int rows, bool norm) {
+    if (rows < (norm ? 3 : 5) || weight_rows < (norm ? 4096 : 8192) || in_width < (norm ? 352 : 1024))
+        return 0;
+    int b = rows <= 4 ? 4 : rows <= 8 ? 8 : 16;
+    while (b > 4 && 4L * b * in_width > kF32BatchLds) b /= 2;
+    if (4L * b * in_width > kF32BatchLds || (!norm && b < 8)) return 0;
+    if (b < 16) return b;
+    const int groups = (rows + 15) / 16;
+    const bool pays = norm ? (long)in_width * rows >= 8192L * groups
+                           : weight_rows >= 16384 || (rows + 3) / 4 == 4 * groups;
+    return pays ? b : 0;
+}
+
 // Whether gemv() can write router logit partials for p (router fields
 // aside), and how many partials per expert it then writes.
 bool gemv_router_ok(const GemvParams &p);
