@@ -15,10 +15,12 @@
 // A launch covers a table of independent tasks (one per active routed expert
 // plus the shared expert, or one dense matrix).  Tiles are 128 token rows x
 // 256 weight rows (SwiGLU pairs: 128 gate + 128 matching up rows, 128
-// outputs), or 32 token rows x 256 weight rows where a launch's tasks hold
+// outputs), or 64 or 32 token rows x 256 weight rows where a launch's tasks hold
 // few rows each; the tile order groups 4 row tiles of a task so that consecutive
 // workgroups on one XCD share weight tiles in that XCD's L2.
 #pragma once
+
+#include <algorithm>
 
 #include "gemv_impl.h"
 
@@ -102,6 +104,33 @@ struct QGemmLaunch {
 int quantize_activations(const float *x, long x_stride, int rows, int width, const float *norm_w,
                          float eps, int8_t *q, float *scale, hipStream_t stream);
 
+// Tile kinds: the weight-streaming tile with 16 token rows, the LDS tiles
+// with 32, 64 or 128.
+enum TileKind { kTileStream16 = 0, kTileLds32 = 1, kTileLds64 = 2, kTileLds128 = 3 };
+
+inline int tile_bm(int kind) {
+    return kind == kTileStream16 ? 16
+           : kind == kTileLds32  ? kQgBMSmall
+           : kind == kTileLds64  ? kQgBMMid
+                                 : kQgBM;
+}
+
+inline int host_tiles(bool dual, int rows, int n_out, int bm) {
+    const int outw = dual ? kQgBW / 2 : kQgBW;
+    return ((rows + bm - 1) / bm) * ((n_out + outw - 1) / outw);
+}
+
+// Dense projections: the smallest tile that covers the matrix in one round of
+// the CUs, else 128 rows.  Tiles of 32 / 64 / 128 rows: 2048 x 2048 at 600 rows
+// 19.8 / 23.9 / 36.4 us, at 1200 rows 36.8 / 27.5 / 39.1, at 2048 rows 42.4 /
+// 31.1 / 45.0; 3648 x 2048 at 600 rows 34.9 / 25.0 / 37.9, at 1200 rows 52.2 /
+// 48.0 / 41.0, at 2048 rows 76.4 / 57.8 / 48.6.
+inline int dense_tile(int rows, bool k128, int n_out, bool dual) {
+    if (k128 && rows <= 16) return kTileStream16;
+    if (host_tiles(dual, rows, n_out, kQgBMSmall) <= 256) return kTileLds32;
+    return host_tiles(dual, rows, n_out, kQgBMMid) <= 256 ? kTileLds64 : kTileLds128;
+}
+
 // One dense task, e.g. a prefill projection.  Epilogue: plain or residual
 // (task.resid) or SwiGLU pair (dual, task.w2 = up).
 int qgemm_single(int fmt, bool dual, const GemmTask &task, hipStream_t stream);
@@ -112,6 +141,12 @@ int qgemm_single(int fmt, bool dual, const GemmTask &task, hipStream_t stream);
 // for shapes it does not take; with `name` set it launches nothing and stores
 // the kernel's template name.
 bool gemv_tiles(const GemvParams &p, hipStream_t stream, std::string *name = nullptr);
+// Token rows of one of its launches: what the scratch for their limbs holds.
+constexpr long kTilesBytes = 64L << 20;
+constexpr int kTilesRows = 8192;
+inline long tiles_chunk(long rows, int width) {
+    return std::min({rows, (long)kTilesRows, kTilesBytes / limb_row_block<4>(width) * 8});
+}
 
 // MoE prefill: builds the per-expert task tables from the device route tables
 // and runs both expert stages for all active experts plus the shared expert.

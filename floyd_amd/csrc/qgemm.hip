@@ -822,7 +822,6 @@ __global__ __launch_bounds__(256, 2) void qgemm_stream_kernel(QGemmLaunch L) {
         const int logical = (lane % kChunks) ^ (j & (kChunks - 1));
         dma_src[d] = row + logical * 16;
     }
-    const int nsteps = tk.k / 128;  // k % 64 == 0; an odd last half-step is handled below
     const int nk = tk.k / 64;
     i32x4 ra[S][2][kLimbs][MB];
     auto issue = [&](int step, int st) {
@@ -890,7 +889,6 @@ __global__ __launch_bounds__(256, 2) void qgemm_stream_kernel(QGemmLaunch L) {
         }
     };
     const int steps = (nk + 1) / 2;  // the last step may hold one slice
-    (void)nsteps;
 #pragma unroll
     for (int j = 0; j < S; ++j)
         if (j < steps) issue(j, j);
@@ -1007,22 +1005,6 @@ static void launch_stream_mb(int fmt, bool dual, const QGemmLaunch &L, int grid,
     }
 }
 
-// Tile kinds: the weight-streaming tile with 16 token rows, the LDS tiles
-// with 32, 64 or 128.
-enum TileKind { kTileStream16 = 0, kTileLds32 = 1, kTileLds64 = 2, kTileLds128 = 3 };
-
-static int tile_bm(int kind) {
-    return kind == kTileStream16 ? 16
-           : kind == kTileLds32  ? kQgBMSmall
-           : kind == kTileLds64  ? kQgBMMid
-                                 : kQgBM;
-}
-
-static int host_tiles(bool dual, int rows, int n_out, int bm) {
-    const int outw = dual ? kQgBW / 2 : kQgBW;
-    return ((rows + bm - 1) / bm) * ((n_out + outw - 1) / outw);
-}
-
 // Tile choices, measured on MI355X.  A batch of at most 16 token rows streams
 // the weights (every task fits one row tile); the streaming tile needs
 // reductions that are whole multiples of 128 (`k128`).
@@ -1037,16 +1019,6 @@ static int moe_tile(int fmt, int rows, double rows_per_expert, bool k128) {
     if (k128 && rows <= 16) return kTileStream16;
     if (fmt == kQ4) return rows_per_expert <= 140.0 ? kTileLds32 : kTileLds128;
     return rows_per_expert <= 32.0 ? kTileLds32 : rows_per_expert <= 64.0 ? kTileLds64 : kTileLds128;
-}
-// Dense projections: the smallest tile that covers the matrix in one round of
-// the CUs, else 128 rows.  Tiles of 32 / 64 / 128 rows: 2048 x 2048 at 600 rows
-// 19.8 / 23.9 / 36.4 us, at 1200 rows 36.8 / 27.5 / 39.1, at 2048 rows 42.4 /
-// 31.1 / 45.0; 3648 x 2048 at 600 rows 34.9 / 25.0 / 37.9, at 1200 rows 52.2 /
-// 48.0 / 41.0, at 2048 rows 76.4 / 57.8 / 48.6.
-static int dense_tile(int rows, bool k128, int n_out, bool dual) {
-    if (k128 && rows <= 16) return kTileStream16;
-    if (host_tiles(dual, rows, n_out, kQgBMSmall) <= 256) return kTileLds32;
-    return host_tiles(dual, rows, n_out, kQgBMMid) <= 256 ? kTileLds64 : kTileLds128;
 }
 
 static int launch_qgemm_fmt(int fmt, bool dual, int kind, const QGemmLaunch &L, int tiles_bound,
@@ -1086,8 +1058,6 @@ int qgemm_single(int fmt, bool dual, const GemmTask &task, hipStream_t stream) {
 // stream, and a call's launches are queued under a lock, so no other call's
 // come between them; wider batches run in row chunks.  (No allocation: a call
 // may be captured.)
-constexpr long kTilesBytes = 64L << 20;
-constexpr int kTilesRows = 8192;
 constexpr int kTilesMaxWidth = 65536;  // the shares' doubles are exact to here
 static_assert(kTilesMaxWidth <= kQgMaxK, "int32 sums");
 __device__ int8_t tiles_limbs[kTilesBytes];
@@ -1152,11 +1122,6 @@ __global__ __launch_bounds__(256) void quantize4_kernel(const float *x, long x_s
     }
 }
 
-// Token rows of one launch.
-static long tiles_chunk(const GemvParams &p) {
-    return std::min<long>(std::min<long>(kTilesRows, kTilesBytes / limb_row_block<4>(p.I) * 8), p.rows);
-}
-
 // Shares of the reduction: as many as keep the launch in one round of the CUs
 // (a 2048-row matrix has 8 tiles per 64 token rows), none shorter than
 // kSplitMinSlices slices (2048 columns), where storing and adding the shares (128
@@ -1180,7 +1145,7 @@ bool gemv_tiles(const GemvParams &p, hipStream_t stream, std::string *name) {
     if (name) {
         char buf[64];
         snprintf(buf, sizeof(buf), "mlh::qgemm_kernel<%d, %s, %d, 4, %s>", p.fmt,
-                 dual ? "true" : "false", kQgBMMid, tile_splits(p, tiles_chunk(p)) > 1 ? "true" : "false");
+                 dual ? "true" : "false", kQgBMMid, tile_splits(p, tiles_chunk(p.rows, p.I)) > 1 ? "true" : "false");
         *name = buf;
         return true;
     }
@@ -1195,7 +1160,7 @@ bool gemv_tiles(const GemvParams &p, hipStream_t stream, std::string *name) {
         (void)hipGetLastError();  // not sticky: the caller falls back
         return false;
     }
-    const long chunk = tiles_chunk(p);
+    const long chunk = tiles_chunk(p.rows, p.I);
     for (long r0 = 0; r0 < p.rows; r0 += chunk) {
         const int n = (int)std::min<long>(chunk, p.rows - r0);
         hipLaunchKernelGGL(quantize4_kernel, dim3(n), dim3(256), 0, stream, p.x + r0 * p.x_stride,
@@ -1307,7 +1272,7 @@ __device__ __forceinline__ void moe_schedule_body(const MoeScheduleParams &sp,
             a.n_out = p.shared_width;
             a.k = p.hidden;
             a.a = p.xq;
-                a.a_scale = p.xq_scale;
+            a.a_scale = p.xq_scale;
             a.a_width = p.hidden;
             a.y = p.shared_hidden;
             a.y_stride = p.shared_width;

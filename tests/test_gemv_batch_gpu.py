@@ -3,9 +3,10 @@ width, from 2 token rows where the one-pass kernels of gemv_mfma.hip do not take
 the shape; gemv_f32_batch.hip; the GEMM tiles of larger batches) against the CPU
 oracle, at the edges of their tiles.
 
-Tolerance: x is split exactly to 30 bits and every product is exact, so the
-difference is the oracle's own serial fp32 sum: at most I * 2^-24 relative, in
-practice sqrt(I) * 2^-24 = 6e-6 at the widest row here.
+Tolerance: x is cut to 30 bits of the largest of its range (ragged widths and
+unaligned operands: fp32) and the limbs' products are exact, so the difference is
+the oracle's own serial fp32 sum: at most I * 2^-24 relative, in practice sqrt(I) *
+2^-24 = 6e-6 at the widest row here.
 """
 import numpy as np
 import pytest
@@ -49,8 +50,8 @@ def test_batch_matches_oracle(device, fmt, out_width, in_width, rows):
 
 # the four-limb GEMM tiles (qgemm.hip) that larger batches take: row tiles of 64
 # and column tiles of 256 with remainders, widths that end inside a 128-wide
-# slice, and a width whose rows take more than one scratch chunk; reductions in 2
-# shares, the last of them ending inside a slice, and in 5
+# slice; reductions in 2 shares, the last of them ending inside a slice, and in 5
+# (rows past one launch's scratch: test_gemm_tiles.py)
 @pytest.mark.parametrize("fmt", [1, 2])
 @pytest.mark.parametrize("out_width,in_width,rows", [
     (11264, 2048, 97), (4100, 64, 300), (3001, 2112, 321), (900, 192, 1100), (5000, 16448, 260),
@@ -78,9 +79,9 @@ def check(fmt, out_width, in_width, rows):
         assert rel_l2(got, res + expect if resid else expect) < TOL
 
 
-# f32 matrices of many rows: token tiles of 4, 8 and 16 with remainders, weight
-# tiles of 64 and 32 with remainders, rows of fewer and more chunks than a
-# wave's two loads, widths whose token rows fill the LDS
+# f32 matrices of many rows on either side of the line between the batch and the
+# vector kernel (narrow ones and 17 rows: vector; the batch kernel's tiles and
+# its line: test_f32_batch.py)
 @pytest.mark.parametrize("out_width,in_width,rows,norm", [
     (4096, 2048, 3, True), (4099, 4, 4, True), (8200, 252, 5, False), (8193, 260, 8, False),
     (9001, 516, 9, True), (8192, 2048, 17, False), (4100, 4096, 12, True), (4097, 9216, 4, True)])

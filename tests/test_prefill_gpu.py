@@ -1,14 +1,15 @@
-"""GPU parity of the prefill path: batches of >= 16 token rows (>= 5 in the
-MoE layer) run every q8/q4 matmul on the int8-limb MFMA GEMM
-(floyd_amd/csrc/qgemm.hip), in 32-row tiles where the tasks hold few rows and
-128-row tiles otherwise, and route through the multi-workgroup routing kernels
-when rows * top_k > 1024.
+"""GPU parity of the prefill path: the MoE layer from 3 token rows and the dense
+projections of larger batches run on the int8-limb MFMA GEMM
+(floyd_amd/csrc/qgemm.hip), smaller projections on the batch matmul
+(gemv_batch.hip; each tile with its own rows: test_gemm_tiles.py), and batches of
+rows * top_k > 1024 route through the multi-workgroup routing kernels.
 
   test_tiny_moe_gemm         one MoE layer at 5, 40 and 200 rows, top-k routing,
                              three format mixes (tests/test_moonlight_metal_moe.c
                              semantics)
-  test_tiny_prefill_gemm     a 40-token prefill through every GEMM path (q/kv_a,
-                             o_proj, dense SwiGLU + down, experts) vs orc_forward
+  test_tiny_prefill_gemm     a 40-token prefill through every matmul (q/kv_a, o_proj
+                             and dense SwiGLU + down on the batch matmul, experts
+                             on the GEMM) vs orc_forward
   test_tiny_prefill_expanded the attention on expanded per-head keys and
                              values (100 + 70 rows) vs orc_attention and
                              orc_forward
@@ -230,7 +231,7 @@ DENSE = [("model.layers.3.self_attn.q_proj.weight", 2048, 3072, 512),
          ("model.layers.3.self_attn.kv_a_proj_with_mqa.weight", 2048, 576, 511),
          ("model.layers.3.self_attn.o_proj.weight", 2048, 2048, 512),
          ("model.layers.0.mlp.down_proj.weight", 11264, 2048, 90),
-         # few rows: the weight-streaming tiles (16 and 32 token rows)
+         # few rows (as kv_a and the down projection above: the batch matmul)
          ("model.layers.3.self_attn.q_proj.weight", 2048, 3072, 16),
          ("model.layers.3.self_attn.kv_a_proj_with_mqa.weight", 2048, 576, 27),
          ("model.layers.0.mlp.down_proj.weight", 11264, 2048, 31)]
@@ -281,8 +282,8 @@ def test_gemm_outliers_moe(moon):
 
 @pytest.mark.parametrize("rows", [511, 512])
 def test_moonlight_prefill_attention(moon, rows):
-    """Prefill MLA (flash form over 16-key tiles, two query rows per
-    workgroup) at 16 heads / latent 512 / rope 64 against orc_attention
+    """Prefill MLA (the expanded form) at 16 heads / latent 512 / rope 64
+    against orc_attention
     (moonlight_kernels.metal:218-375 with key_count = pos + r + 1); then
     prefill(n - 1) + decode(1) equals prefill(n) on the last row
     (tests/test_moonlight_metal_mla.c:219-238)."""

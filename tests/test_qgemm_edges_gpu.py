@@ -34,7 +34,8 @@ def edge(request, device, tmp_path_factory):
 
 
 # streaming tile (k a multiple of 128) or 32-row tile, 32-row tiles with one
-# and several row tiles per expert, 128-row tiles (over 80 rows per expert)
+# and several row tiles per expert, and for q8 64-row tiles (400 rows: over 32 rows
+# per expert) and 128-row tiles (1000 rows: over 64); q4 stays on 32 rows here
 @pytest.mark.parametrize("rows", [3, 17, 61, 400, 1000])
 def test_moe_block_edges(edge, rows):
     cfg, tensors, model, bits = edge
