@@ -337,15 +337,12 @@ int gemv(const GemvParams &p_in, hipStream_t stream) {
         return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
     if (!off_batch(p_in, vector_ok) && gemv_batch(p_in, !vector_ok, stream))
         return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
-    // token rows beyond 4 run as slices of 4 (register budget) along grid.y
-    // of one launch
+    // one row, or f32: token rows beyond 4 run as slices of 4 (register budget)
+    // along grid.y of one launch
     bool done = false;
     if (vector_ok) {
         int plan_rows = p_in.rows < kMaxGemvRows ? p_in.rows : kMaxGemvRows;
         if (plan_rows == 3) plan_rows = 4;  // the kernel takes 1, 2 or 4 token rows
-        // the quantised x rows of a workgroup must fit its LDS
-        while (plan_rows > 1 && gemv_lds_bytes_rt(p_in.fmt, plan_rows, p_in.I) > kMaxGemvLds)
-            plan_rows /= 2;
         const GemvPlan plan = plan_gemv(p_in.fmt, p_in.O, p_in.I, plan_rows,
                                         p_in.epilogue == kEpiSiluDual);
         GemvLaunch L;

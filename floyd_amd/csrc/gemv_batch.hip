@@ -47,6 +47,7 @@
 // 120 / 18; 11999 x 11999 at 1 row 189 / 126, at 16 rows 1769 / 143.
 #include "limb_split.h"
 
+#include <algorithm>
 #include <cstdio>
 #include <string>
 
@@ -561,7 +562,6 @@ bool gemv_batch(const GemvParams &p, bool fp32x, hipStream_t stream, std::string
     if ((p.fmt != kQ8 && p.fmt != kQ4) || p.limbs || p.router_parts) return false;
     const bool dual = p.epilogue == kEpiSiluDual;
     const BatchPlan pl = plan_batch(p, fp32x);
-    if (pl.grid.z > 65535) return false;
     if (name) {
         char buf[96];
         snprintf(buf, sizeof(buf),
@@ -570,12 +570,21 @@ bool gemv_batch(const GemvParams &p, bool fp32x, hipStream_t stream, std::string
         *name = buf;
         return true;
     }
-    if (p.fmt == kQ8) {
-        if (dual) launch_tok<kQ8, true>(p, pl, stream);
-        else launch_tok<kQ8, false>(p, pl, stream);
-    } else {
-        if (dual) launch_tok<kQ4, true>(p, pl, stream);
-        else launch_tok<kQ4, false>(p, pl, stream);
+    const int slice = 65535 * pl.tok;  // token rows of a launch's grid
+    for (long r0 = 0; r0 < p.rows; r0 += slice) {
+        GemvParams q = p;
+        q.rows = (int)std::min<long>(slice, p.rows - r0);
+        q.x += r0 * p.x_stride;
+        q.y += r0 * p.y_stride;
+        if (p.resid) q.resid += r0 * p.resid_stride;
+        const BatchPlan ql = plan_batch(q, fp32x);
+        if (p.fmt == kQ8) {
+            if (dual) launch_tok<kQ8, true>(q, ql, stream);
+            else launch_tok<kQ8, false>(q, ql, stream);
+        } else {
+            if (dual) launch_tok<kQ4, true>(q, ql, stream);
+            else launch_tok<kQ4, false>(q, ql, stream);
+        }
     }
     return true;
 }

@@ -1153,10 +1153,10 @@ template <int FMT>
 bool dispatch_gemv_fmt(const GemvLaunch &L, int mode, const GemvPlan &plan, dim3 grid,
                        hipStream_t stream) {
     if (mode == 0) {
-        switch (plan.b) {
-        case 1: return dispatch_gemv_b<0, FMT, 1>(L, plan, grid, stream);
-        case 2: return dispatch_gemv_b<0, FMT, 2>(L, plan, grid, stream);
-        case 4: return dispatch_gemv_b<0, FMT, 4>(L, plan, grid, stream);
+        if (plan.b == 1) return dispatch_gemv_b<0, FMT, 1>(L, plan, grid, stream);
+        if constexpr (FMT == kF32) {  // q8 / q4 of several rows: gemv_batch.hip
+            if (plan.b == 2) return dispatch_gemv_b<0, FMT, 2>(L, plan, grid, stream);
+            if (plan.b == 4) return dispatch_gemv_b<0, FMT, 4>(L, plan, grid, stream);
         }
         return false;
     }

@@ -67,6 +67,27 @@ def test_tile_rows_stay_within_31_bit_offsets(fmt, swiglu):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("in_width", [16, 19])
+def test_more_rows_than_one_grid(device, in_width):
+    """The batch kernel's grid holds 65535 token tiles of 16: more rows run in
+    slices, each with its own rows of x, y and the residual."""
+    rows, out_width = 16 * 65535 + 21, 3
+    print(f"[gpu] O={out_width} I={in_width} rows={rows}", flush=True)
+    assert "gemv_batch" in native.gemv_kernel_name(1, out_width, in_width, rows)
+    rng = np.random.default_rng(4)
+    q = rng.integers(-127, 128, (out_width, in_width), dtype=np.int8)
+    s = np.full(out_width, 1.0 / 127, np.float32)
+    x = rng.standard_normal((rows, in_width)).astype(np.float32)
+    res = rng.standard_normal((rows, out_width)).astype(np.float32)
+    dq, ds, dx, dr = (DeviceBuffer.from_array(a) for a in (q.view(np.uint8), s, x, res))
+    dy = DeviceBuffer(rows * out_width * 4)
+    native.gemv(1, dq, ds, dx, dy, out_width, in_width, rows, resid=dr)
+    expect = x.astype(np.float64) @ q.T.astype(np.float64) / 127 + res
+    # at most 24 roundings, of sums below 100
+    assert np.abs(dy.download(np.float32).reshape(rows, out_width) - expect).max() < 24 * 100 * 2.0 ** -24
+
+
+@pytest.mark.gpu
 def test_outputs_of_over_2_gib(device):
     """64 token rows of 8,388,700 outputs, every output against numpy's fp32
     product (64 columns: at most 64 roundings of 2^-24 each of the sum of the
