@@ -5,8 +5,9 @@
 // RMSNorm / residual / SwiGLU variants, :23-41, :533-541).
 //
 // Numerics: those of gemv_mfma.hip.  A wave splits its 256-column range of a
-// token row (a part of it, below) into four exact int8 limbs against a
-// power-of-two step that maps the range's largest |x| below 2^30, the products
+// token row (a part of it, below) into four int8 limbs against a power-of-two
+// step that maps the range's largest |x| below 2^30 (what lies below the step is
+// cut: columns 2^6 and more below the largest keep fewer than 24 bits), the products
 // with the stored weights are exact int32 sums, and the ranges' sums are added
 // in fp32.  A NaN or infinity in the range makes the token row's outputs NaN.
 //

@@ -1,5 +1,6 @@
-// limb_split.h -- the exact four-limb int8 split of fp32 values that the
-// matrix-core GEMV kernels share (gemv_mfma.hip, gemv_batch.hip).
+// limb_split.h -- the four-limb int8 split of fp32 values (30 bits of the largest
+// of a range) that the matrix-core GEMV kernels share (gemv_mfma.hip,
+// gemv_batch.hip, the four-limb tiles of qgemm.hip).
 #pragma once
 
 #include "mlh_device.h"

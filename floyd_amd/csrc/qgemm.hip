@@ -10,9 +10,9 @@
 //
 // Bound: the copies (the layer without products 457 us, without copies 474, at
 // 583 in all for q8 at T = 2048) and the card's power limit (the same launches
-// on zero activations: 495 us).  Whole MoE layer on MI355X, T = 2048: q8 653 ->
-// 556 us, q4 618 -> 543; T = 600: q8 323 -> 296, q4 278 -> 225; T = 64: q8 158
-// -> 154, q4 136 -> 121 (64-wide q8 slices by flat LDS DMA, q4 slices unpacked
+// on zero activations: 495 us).  Whole MoE layer on MI355X, T = 2048: q8 655 ->
+// 562 us, q4 616 -> 548; T = 600: q8 317 -> 276, q4 275 -> 225; T = 64: q8 161
+// -> 159, q4 128 -> 118 (64-wide q8 slices by flat LDS DMA, q4 slices unpacked
 // through registers, limb planes and a read-wait-multiply order before).
 // MFMA operand layout (measured on gfx950): lane l supplies row (l % 32) and
 // the 16-byte k chunk (l / 32) of a 32-wide k step, for A rows and for B
