@@ -290,7 +290,7 @@ static bool off_batch(const GemvParams &p, bool vector_ok) {
 }
 
 // Template name of the kernel gemv() launches for this shape (aligned
-// operands, no pre-split x).
+// operands).
 std::string gemv_kernel_name(int fmt, int O, int I, int rows, bool dual) {
     GemvParams q;
     q.fmt = fmt;

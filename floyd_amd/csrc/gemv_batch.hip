@@ -555,12 +555,12 @@ void launch_tok(const GemvParams &p, const BatchPlan &pl, hipStream_t stream) {
 
 }  // namespace
 
-// Launches the kernel for p (q8 / q4, no pre-split x, no router partials), with
+// Launches the kernel for p (q8 / q4, no router partials), with
 // x in fp32 (FP32X) or, where the vector kernel takes p, in limbs; false,
 // launching nothing, when it does not take it.  With `name` set it
 // launches nothing and stores the kernel's template name.
 bool gemv_batch(const GemvParams &p, bool fp32x, hipStream_t stream, std::string *name) {
-    if ((p.fmt != kQ8 && p.fmt != kQ4) || p.limbs || p.router_parts) return false;
+    if ((p.fmt != kQ8 && p.fmt != kQ4) || p.router_parts) return false;
     const bool dual = p.epilogue == kEpiSiluDual;
     const BatchPlan pl = plan_batch(p, fp32x);
     if (name) {

@@ -143,7 +143,7 @@ void launch(const GemvParams &p, hipStream_t stream) {
 // nothing and stores the kernel's template name.
 bool gemv_f32_batch(const GemvParams &p, hipStream_t stream, std::string *name) {
     auto al = [](const void *q) { return ((uintptr_t)q & 15u) == 0; };
-    if (p.fmt != kF32 || p.epilogue == kEpiSiluDual || p.limbs || p.router_parts || p.I % 4 ||
+    if (p.fmt != kF32 || p.epilogue == kEpiSiluDual || p.router_parts || p.I % 4 ||
         !al(p.w) || !al(p.x) || p.x_stride % 4 || (p.norm_w && !al(p.norm_w)))
         return false;
     const int b = f32_batch_rows(p.O, p.I, p.rows, p.norm_w != nullptr);

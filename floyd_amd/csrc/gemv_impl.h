@@ -901,7 +901,7 @@ __global__ __launch_bounds__(W * 64) void gemv_kernel(GemvLaunch L) {
             job.x[b] = p.x + r * p.x_stride;
             job.y[b] = p.y + r * p.y_stride;
             job.resid[b] = p.resid ? p.resid + r * p.resid_stride : nullptr;
-            job.limbs[b] = p.limbs ? p.limbs + r * p.limb_stride : nullptr;
+            job.limbs[b] = nullptr;
         }
         job.norm_w = p.norm_w;
         job.eps = p.eps;

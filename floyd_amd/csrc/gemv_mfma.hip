@@ -928,7 +928,7 @@ __global__ __launch_bounds__(1024) void gemv_mfma_wide_kernel(GemvParams p) {
 // unevenly over the CUs) 8.52 against 8.28, which stays on split-k.
 bool wide_ok(const GemvParams &p) {
     return (p.fmt == kQ8 || p.fmt == kQ4) && p.rows == 1 && p.epilogue != kEpiSiluDual &&
-           !p.limbs && !p.router_parts && p.I > 4096 && p.I <= 1024 * kWideMaxWaves &&
+           !p.router_parts && p.I > 4096 && p.I <= 1024 * kWideMaxWaves &&
            p.I % 1024 == 0 && (p.O == 2048 || p.O == 4096);
 }
 template <int FMT>
@@ -974,7 +974,7 @@ int splitk_splits(const GemvParams &p) {
     const int chunk = 4 * kSkQuarter;
     const int splits = (p.I + chunk - 1) / chunk;
     if ((p.fmt != kQ8 && p.fmt != kQ4) || p.epilogue == kEpiSiluDual || p.rows < 1 ||
-        p.rows > 4 || p.rows == 3 || p.limbs || p.router_parts || p.I <= 4096 || p.O > 4096 ||
+        p.rows > 4 || p.rows == 3 || p.router_parts || p.I <= 4096 || p.O > 4096 ||
         p.I % kSkQuarter || splits > kSkMaxSplits || (p.O + kRows - 1) / kRows > kSkMaxRowBlocks)
         return 0;
     return splits;
@@ -1073,8 +1073,7 @@ bool launch_b(const MfmaGemvArgs &a, hipStream_t stream, std::string *name) {
 }  // namespace
 
 // The matrix-core GEMV for the shapes it covers (q8 / q4, 1, 2 or 4 token
-// rows, I a multiple of 256 (q8) or 512 (q4), aligned operands, no pre-split
-// x); returns false, launching nothing, otherwise.  Measured on MI355X
+// rows, I a multiple of 256 (q8) or 512 (q4), aligned operands); returns false, launching nothing, otherwise.  Measured on MI355X
 // against the vector kernel (gemv_impl.h), graph replays: q4 11264 x 2048
 // 5.27 against 5.95 us, q8 3648 x 2048 4.16 against 4.72 us, q8 11264 x 2048
 // at 4 rows 9.9 against 12.7 us.  Wide-k matrices with few rows (2048 x
@@ -1085,7 +1084,7 @@ bool launch_b(const MfmaGemvArgs &a, hipStream_t stream, std::string *name) {
 // Output rows per workgroup when the matrix-core kernels take p (operand
 // alignment checked when `aligned`), else 0.
 static int mfma_rows(const GemvParams &p, bool aligned) {
-    if ((p.fmt != kQ8 && p.fmt != kQ4) || p.rows < 1 || p.rows > 4 || p.rows == 3 || p.limbs)
+    if ((p.fmt != kQ8 && p.fmt != kQ4) || p.rows < 1 || p.rows > 4 || p.rows == 3)
         return 0;
     const bool dual = p.epilogue == kEpiSiluDual;
     const int rw = p.O < 4096 && p.I > 4096 ? 8 : kRows;

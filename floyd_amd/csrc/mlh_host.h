@@ -35,11 +35,6 @@ struct GemvParams {
     const float *resid = nullptr;  // kEpiResidual: y = resid + result
     long resid_stride = 0;
     int epilogue = kEpiPlain;
-    // optional (q8 / q4): x already split into limb rows (limb_quantise_rows,
-    // same format and width), row stride limb_stride bytes; norm_w is then
-    // already applied
-    const unsigned char *limbs = nullptr;
-    long limb_stride = 0;
     // optional, one token row of a plain or residual epilogue on the int8
     // matrix-core kernels (gemv_router_ok): router logit partials of the
     // output row y for the next MoE layer's router.  Workgroup j of the

@@ -1138,7 +1138,7 @@ static int tile_splits(const GemvParams &p, long rows) {
 bool gemv_tiles(const GemvParams &p, hipStream_t stream, std::string *name) {
     const bool dual = p.epilogue == kEpiSiluDual;
     auto al = [](const void *v) { return ((uintptr_t)v & 15u) == 0; };
-    if (!qgemm_shape_ok(p.fmt, p.I) || p.I > kTilesMaxWidth || p.limbs || p.router_parts || !al(p.w) ||
+    if (!qgemm_shape_ok(p.fmt, p.I) || p.I > kTilesMaxWidth || p.router_parts || !al(p.w) ||
         (dual && !al(p.w2)) || !al(p.x) || p.x_stride % 4 || (p.norm_w && !al(p.norm_w)) ||
         p.y_stride > kQgMaxStride || (p.resid && p.resid_stride > kQgMaxStride))
         return false;
