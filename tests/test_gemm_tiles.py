@@ -168,6 +168,27 @@ def test_rows_past_the_scratch(device, fmt, out_width, in_width, rows):
         assert (np.abs(got - expect) <= bound).all()
 
 
+# reductions shared by several workgroups, whose counters and shares are the
+# library's own: the batch kernel (limbs and fp32) and the tiles
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt,out_width,in_width,rows", [
+    (1, 576, 11264, 20), (2, 40, 6145, 20), (1, 2048, 4160, 210)])
+def test_replays_repeat_the_eager_call(device, fmt, out_width, in_width, rows):
+    print(f"[gpu] graph replays fmt={fmt} O={out_width} I={in_width} rows={rows}", flush=True)
+    q, s = make_weights(fmt, out_width, in_width, seed=out_width + in_width)
+    x = O.fill_normal(rows * in_width, 31 + rows)
+    dq, ds, dx = (DeviceBuffer.from_array(a) for a in (q, s, x))
+    eager, dy = DeviceBuffer(rows * out_width * 4), DeviceBuffer(rows * out_width * 4)
+    native.gemv(fmt, dq, ds, dx, eager, out_width, in_width, rows)
+    expect = eager.download(np.float32)
+    for launches in (1, 4):  # per replay; each graph is replayed twice
+        dy.zero()
+        native.time_gemv(fmt, [dq], [ds], dx, dy, out_width, in_width, rows, 1, launches)
+        np.testing.assert_array_equal(dy.download(np.float32), expect)
+        native.gemv(fmt, dq, ds, dx, eager, out_width, in_width, rows)
+        np.testing.assert_array_equal(eager.download(np.float32), expect)
+
+
 @pytest.mark.gpu
 def test_moe_128_row_tile(moon):
     """Experts of more than 140 rows each on average (1601 rows of 6 experts): the
